@@ -1760,6 +1760,30 @@ static int verify_pass(g4v_ctx* c, const int* toks, int na, int nb, int pos0, in
 // a linear layer of a prefill segment: lin_multi / lin1 (E:310-317) take W4A8 when the block has
 // M >= 2 rows (G_I8_ACTIVE during prefill), else the exact-float GEMV.  quant = false reuses the
 // quantised rows of the previous call (same x).
+//
+// the exact-float products of more than MAXM rows over the W4A8 operand tiles (the matrix-core
+// GEMM, g4v_gemmx.hip; every model matrix has N % 16 == 0); false: at most MAXM rows, the GEMV's.  The
+// group sums sit in the W4A8 row scales' buffer (both [rows][K/32] floats, one of the two in use).
+static bool pf_exact(g4v_ctx* c, int n, const Mat* const* m, const float* x, int M, float* const* y, bool gateup) {
+  if (M <= MAXM) return false;
+  constexpr int R = 65536;  // rows a launch (its 32-bit offsets reach 2^30 floats of x; K <= 12288)
+  for (int r = 0; r < M; r += R) {
+    GemmXArgs a{};
+    for (int j = 0; j < n; ++j) {
+      a.tw[j] = m[j]->a8w.as<uint4>();
+      a.ts[j] = m[j]->a8s.as<uint4>();
+      a.y[j] = y[j] + (size_t)r * m[j]->N;
+      a.ldy[j] = a.N[j] = m[j]->N;
+    }
+    a.ldx = a.K = m[0]->K;
+    a.x = x + (size_t)r * a.K;
+    a.gs = c->pfsx.as<float>();
+    a.M = std::min(R, M - r);
+    if (!launch_gemm_x(a, n, gateup, c->st)) return false;
+  }
+  return true;
+}
+
 static void pf_lin(g4v_ctx* c, const Mat& m, const float* x, int M, float* y, bool i8, bool quant) {
   if (i8) {
     if (quant)
@@ -1767,13 +1791,13 @@ static void pf_lin(g4v_ctx* c, const Mat& m, const float* x, int M, float* y, bo
                         nullptr, nullptr, nullptr, c->st);
     launch_w4a8_gemm(m.a8w.as<uint4>(), m.a8s.as<uint4>(), c->pfxq.as<uint16_t>(), c->pfsx.as<float>(),
                      c->pfcorr.as<float>(), y, M, m.N, m.K, m.N, c->st);
-  } else {  // the exact-float GEMV, MAXM rows a launch (each row's result is independent of the others)
-    for (int r = 0; r < M; r += MAXM)
-      launch_gemv(plain_args(m, x + (size_t)r * m.K, y + (size_t)r * m.N, std::min(MAXM, M - r)), EPI_STORE, c->st);
+  } else {  // exact float: the matrix-core GEMM past MAXM rows, else the GEMV
+    const Mat* mp = &m;
+    if (!pf_exact(c, 1, &mp, x, M, &y, false)) launch_gemv(plain_args(m, x, y, M), EPI_STORE, c->st);
   }
 }
 
-// up to three products of the same input (same K) in one launch per MAXM rows: q / k / v, gate / up
+// up to three products of the same input (same K) in one launch: q / k / v, gate / up
 static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x, int M, float* const* y, bool i8) {
   if (i8) {
     bool n16 = true;
@@ -1797,20 +1821,28 @@ static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x,
     for (int j = 0; j < n; ++j) pf_lin(c, *m[j], x, M, y[j], true, j == 0);
     return;
   }
-  const int K = m[0]->K;
-  for (int r = 0; r < M; r += MAXM) {
-    GemvArgs a{};
-    for (int j = 0; j < n; ++j) {
-      a.mat[j] = m[j]->dev();
-      a.y[j] = y[j] + (size_t)r * m[j]->N;
-      a.ldy[j] = m[j]->N;
-    }
-    a.x = x + (size_t)r * K;
-    a.ldx = K;
-    a.K = K;
-    a.M = std::min(MAXM, M - r);
-    launch_gemv(a, EPI_STORE, c->st);
+  if (pf_exact(c, n, m, x, M, y, false)) return;
+  GemvArgs a{};
+  for (int j = 0; j < n; ++j) {
+    a.mat[j] = m[j]->dev();
+    a.y[j] = y[j];
+    a.ldy[j] = m[j]->N;
   }
+  a.x = x;
+  a.ldx = a.K = m[0]->K;
+  a.M = M;
+  launch_gemv(a, EPI_STORE, c->st);
+}
+
+// gate, up and the activation act = r16(r16(gelu8(r16 g)) * r16 u) (E:1363-1371)
+static void pf_gate_up(g4v_ctx* c, const Mat& mg, const Mat& mu, const float* x, int M, float* gb, float* ub,
+                       float* act, bool i8) {
+  const Mat* m[2] = {&mg, &mu};
+  float* ya[2] = {act, act};
+  if (!i8 && pf_exact(c, 2, m, x, M, ya, true)) return;
+  float* yg[2] = {gb, ub};
+  pf_lin_multi(c, 2, m, x, M, yg, i8);
+  launch_pf_act(gb, ub, act, (size_t)M * mg.N, c->st);
 }
 
 static int pf_alloc(g4v_ctx* c, int rows, size_t sfl) {
@@ -1861,9 +1893,11 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
     const int ty = lay.sliding ? 0 : 1;
     uint16_t* KCl = c->KC.as<uint16_t>() + (size_t)l * c->kvcap * HD;
     uint16_t* VCl = c->VC.as<uint16_t>() + (size_t)l * c->kvcap * HD;
-    pf_lin(c, lay.m[0], a, M, q, i8, true);  // E:1289
-    pf_lin(c, lay.m[1], a, M, k, i8, false);
-    pf_lin(c, lay.m[2], a, M, v, i8, false);
+    {  // E:1289
+      const Mat* mq[3] = {&lay.m[0], &lay.m[1], &lay.m[2]};
+      float* yq[3] = {q, k, v};
+      pf_lin_multi(c, 3, mq, a, M, yq, i8);
+    }
     const float* cs = c->rope.as<float>() + (size_t)(2 * ty) * c->ctxcap * (HD / 2);
     const float* sn = cs + (size_t)c->ctxcap * (HD / 2);
     launch_pf_qkv(q, k, v, ln.qn, ln.kn, cs, sn, KCl, VCl, P0, M, st);
@@ -1888,9 +1922,7 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
     }
     pf_lin(c, lay.m[3], att, M, o, i8, true);  // E:1356
     launch_pf_post_attn(o, x, a, ln.post_attn, ln.pre_ff, M, st);
-    pf_lin(c, lay.m[4], a, M, gb, i8, true);  // E:1366-1371
-    pf_lin(c, lay.m[5], a, M, ub, i8, false);
-    launch_pf_act(gb, ub, act, (size_t)M * c->I, st);
+    pf_gate_up(c, lay.m[4], lay.m[5], a, M, gb, ub, act, i8);  // E:1366-1371
     pf_lin(c, lay.m[6], act, M, o, i8, true);  // E:1373
     const bool lastl = l + 1 == c->NL;
     launch_pf_post_ff(o, x, a, ln.post_ff, lastl ? nullptr : c->L[l + 1]->ln().in_ln, c->fnorm.as<float>(),
@@ -2075,12 +2107,7 @@ void gm_forward(g4v_ctx* c, int M, int pos0, int nsplit, int sib, int hrow, bool
     if (split) pmark(c, PT_ATTN, 0, 0);
     pf_lin(c, lay.m[3], R.att, M, R.o, i8, true);                       // E:1356
     launch_pf_post_attn(R.o, R.x, R.a, post_attn, pre_ff, M, st);       // E:1358-1361
-    {  // E:1363-1371: gate and up in one launch
-      const Mat* mg[2] = {&lay.m[4], &lay.m[5]};
-      float* yg[2] = {R.g, R.u};
-      pf_lin_multi(c, 2, mg, R.a, M, yg, i8);
-    }
-    launch_pf_act(R.g, R.u, R.act, (size_t)M * G.I, st);
+    pf_gate_up(c, lay.m[4], lay.m[5], R.a, M, R.g, R.u, R.act, i8);  // E:1363-1371
     pf_lin(c, lay.m[6], R.act, M, R.o, i8, true);                                               // E:1373
     launch_pf_post_ff(R.o, R.x, R.a, post_ff, nullptr, nullptr, 1.0f, nullptr, -1, M, st);      // E:1375-1377
     pf_lin(c, G.pg, R.x, M, R.pgv, i8, true);                                                   // E:1379-1384

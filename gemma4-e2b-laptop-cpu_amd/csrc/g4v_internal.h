@@ -314,6 +314,22 @@ int launch_w4a8_dec(const A8Dec& m, int n, const uint16_t* xqb, const float* sxt
                     hipStream_t st);
 void launch_w4a8_gemm(const uint4* tw, const uint4* ts, const uint16_t* xqb, const float* sxt, const float* corr,
                       float* y, int M, int N, int K, int ldy, hipStream_t st);
+// exact-order products of many rows (g4v_gemmx.hip) on the W4A8 operand tiles: up to three matrices
+// of one input x [M][ldx = K] (N_j % 16 == 0, K % 256 == 0), y[j] [M][ldy[j]]; gateup: matrices 0 and
+// 1 are gate and up (the same N) and y[0] receives gelu(gate) * up.  x's rows are K floats;
+// gs: scratch for the group sums, [M][K/32].  Returns 0 (nothing launched) for a shape it does not serve.
+struct GemmXArgs {
+  const uint4* tw[3];
+  const uint4* ts[3];
+  float* y[3];
+  int ldy[3];
+  int N[3];
+  int t0[4];  // set by launch_gemm_x
+  const float* x;
+  const float* gs;
+  int ldx, K, M;
+};
+int launch_gemm_x(const GemmXArgs& a, int nmat, bool gateup, hipStream_t st);
 int w4a8_mpad(int M);  // rows the quantised operand holds for M rows
 
 // prompt lookup (g4v_draft.hip): appends app.t[0 .. app.n) to hist [L0 ..] and writes

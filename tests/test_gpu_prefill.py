@@ -78,6 +78,31 @@ def test_prefill_exact_float_matches_oracle(orc, g4v, n, NL, ctx, pfb, pos0):
         dev.close()
 
 
+# the many-row exact product around its tiles of 32 rows x 32 outputs, and its smallest M (9; 8 rows
+# and fewer take the GEMV); I 256 and 768: gate / up tiles and K of one and three chunk pairs
+@pytest.mark.parametrize("n,I", [(9, 256), (31, 768), (32, 256), (33, 768), (64, 256), (97, 768)])
+def test_prefill_exact_float_row_tiles(orc, g4v, n, I):
+    from oracle import Model
+    V, NL, ctx, seed = 4096, 2, 128, 17
+    toks = np.random.default_rng(n).integers(0, V, n).astype(np.int32)
+    note(f"exact-float row tiles n={n} I={I}")
+    dev = g4v.Device(0)
+    om = Model(orc, seed, V, NL, I, ctx)
+    try:
+        dev.model_synth(seed, V, NL, I, ctx)
+        dev.set_prefill_int8(False)
+        _, hd = dev.prefill(toks, hidden=True)
+        ho = om.prefill(toks, i8=False)
+        assert same(hd, ho), first_diff(hd, ho)
+        for what in ("KC", "VC"):
+            a = dev.read(what, np.uint16).reshape(NL, -1, 256)[:, :n]
+            b = om.get(what, np.uint16, NL * ctx * 256).reshape(NL, ctx, 256)[:, :n]
+            assert same(a, b), (what, first_diff(a.ravel(), b.ravel()))
+    finally:
+        om.close()
+        dev.close()
+
+
 def test_prefill_then_lookup_decode(orc, g4v):
     """a motif prompt, then rounds of prompt-lookup drafts verified as a chain (E:1617-1661)"""
     from oracle import Model
