@@ -301,7 +301,7 @@ __global__ __launch_bounds__(512) void k_gemv_a8p(GemvTArgs a) {
 // LDS: U (the prologue's rows [8][A8_XPS], then A32 [48][CG][8][16]), AQ [48][A8N_QS] uint64 (word h
 // of row m at 8 h + m: a wave's operand reads of one group are 32 consecutive words),
 // SXL [48][8], SWL [CG][6][16] uint4, YL [CG][8][16]
-constexpr int A8_XPS = 1600;  // row stride of the prologue's rows in LDS (16 RMS chains of 100)
+constexpr int A8_XPS = 1600;  // row stride of the prologue's rows in LDS
 constexpr int A8N_QS = 33;    // operand words per group in LDS (32 + 1: the quantisation stores of
                               // consecutive groups on distinct banks)
 template <int CG>
@@ -313,7 +313,8 @@ constexpr size_t a8n_lds() {
   return (size_t)a8n_ufloats<CG>() * 4 + (size_t)48 * A8N_QS * 8 + (size_t)48 * 8 * 4 + (size_t)CG * 6 * 16 * 16 +
          (size_t)CG * 8 * 16 * 4;
 }
-template <int XM, int CG>
+// WPR: waves per row of the norm prologue (2 for up to four rows)
+template <int XM, int CG, int WPR>
 __global__ __launch_bounds__(512) void k_gemv_a8n(GemvTArgs a) {
   constexpr int G = H / 32, GC4 = G / 4, G8 = G / 8, NU = (CG * GC4 + 7) / 8;
   extern __shared__ float4 lds4[];
@@ -357,102 +358,71 @@ __global__ __launch_bounds__(512) void k_gemv_a8n(GemvTArgs a) {
 
   {
     // E:1358-1361 (mode 1) / E:1375-1378 with E:1390-1404 (mode 2) / E:1375-1377 (mode 3: x1 is
-    // the product's input) for row w, as k_gemv_t's norm prologue forms it; the row goes to U in
-    // plain order (stride A8_XPS).  Rows past M are not formed (their operand words are zero).
-    constexpr int RW4 = H / 4, PER = RW4 / 64;
-    const bool live = w < M;
-    const int mr = min(w, M - 1);
-    const float4* o4 = reinterpret_cast<const float4*>(a.nrm_o) + (size_t)mr * RW4 + lane;
-    const float4* x4 = reinterpret_cast<const float4*>(a.nrm_xin) + (size_t)mr * RW4 + lane;
-    const float4* w14 = reinterpret_cast<const float4*>(a.nrm_w1) + lane;
-    const float4* w24 = reinterpret_cast<const float4*>(a.nrm_w2) + lane;
-    float4 ov[PER], xv[PER];
+    // the product's input), as k_gemv_t's norm prologue forms them: row w / WPR on WPR waves.  The
+    // rows go to U in plain order (stride A8_XPS).  Rows past M are not formed (their operand words
+    // are zero).
+    constexpr int RW4 = H / 4, PER = RW4 / 64 / WPR;
+    __shared__ RmsShare SSP[2];
+    const int wq = w / WPR, u0 = lane + 64 * PER * (w % WPR);
+    const bool live = wq < M;
+    const int mr = min(wq, M - 1);
+    const float4* o4 = reinterpret_cast<const float4*>(a.nrm_o) + (size_t)mr * RW4 + u0;
+    const float4* x4 = reinterpret_cast<const float4*>(a.nrm_xin) + (size_t)mr * RW4 + u0;
+    const float4* w14 = reinterpret_cast<const float4*>(a.nrm_w1) + u0;
+    const float4* w24 = reinterpret_cast<const float4*>(a.nrm_w2) + u0;
+    float4 ov[PER], xv[PER], w1[PER], w2[PER];
     if (live) {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         ov[k] = o4[64 * k];
         xv[k] = x4[64 * k];
+        w1[k] = w14[64 * k];
+        if constexpr (XM != 1) w2[k] = w24[64 * k];
       }
     }
     issue_w();
+    const bool after_mlp = a.nrm_mode == 2;
+    const float scal = after_mlp ? a.nrm_scalar : 1.0f;  // (r16(v * 1) = v: no branch per element)
+    auto res1 = [&](float o, float xr, float wt, float r1) { return r16(r16(xr + r16((o * r1) * wt)) * scal); };
+    // the row's elements again, for the rare sum that needs the reference's order
+    auto o_at = [&](int e) { return r16(a.nrm_o[(size_t)mr * H + e]); };
     if (live) {
-      float* XR = U + (size_t)w * A8_XPS;
-      float* CR = XR;  // E:326-345, chains t = e % 16 at 100 t (see k_gemv_t)
-      auto rms_row = [&](const float4 (&v)[PER]) -> float {
 #pragma unroll
-        for (int k = 0; k < PER; ++k) {
-          const float f[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const int e = 4 * (lane + 64 * k) + c;
-            CR[(e & 15) * 100 + (e >> 4)] = f[c];
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        double part = 0;
-        if (lane < 16) {
-          const float4* ch = reinterpret_cast<const float4*>(CR + lane * 100);
-#pragma unroll
-          for (int i = 0; i < H / 64; ++i) {
-            const float4 q = ch[i];
-            const double d0 = (double)q.x, d1 = (double)q.y, d2 = (double)q.z, d3 = (double)q.w;
-            part = fma(d0, d0, part);
-            part = fma(d1, d1, part);
-            part = fma(d2, d2, part);
-            part = fma(d3, d3, part);
-          }
-        }
-        const double b2 = part + shl_d<4>(part);
-        const double c2 = b2 + shl_d<8>(b2);
-        const double d2 = c2 + shl_d<2>(c2);
-        const double e2 = d2 + shl_d<1>(d2);
-        const uint64_t u = as_u64(e2);
-        const double ss = as_f64(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 0) << 32) |
-                                 (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 0));
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        return 1.0f / sqrtf((float)(ss / H) + 1e-6f);
-      };
-      const int nmode = a.nrm_mode;
-      const bool after_mlp = nmode == 2;
-      const float scal = a.nrm_scalar;
-      float4 w1[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) w1[k] = w14[64 * k];
-      float4 os[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) os[k] = make_float4(r16(ov[k].x), r16(ov[k].y), r16(ov[k].z), r16(ov[k].w));
-      const float r1 = rms_row(os);
-      float4 x1[PER];
+      for (int k = 0; k < PER; ++k) ov[k] = make_float4(r16(ov[k].x), r16(ov[k].y), r16(ov[k].z), r16(ov[k].w));
+      share_sumsq(ov, SSP[0], w);
+    }
+    lds_barrier();
+    float r1 = 0.f;
+    float4 x1[PER];
+    float* XR = U + (size_t)wq * A8_XPS;
+    if (live) {
+      r1 = 1.0f / sqrtf(row_mean<WPR>(SSP[0], 4 * WPR * wq, o_at) + 1e-6f);
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
-        const float4 o = os[k], wv = w1[k], xr = xv[k];
-        float4 v = make_float4(r16(xr.x + r16((o.x * r1) * wv.x)), r16(xr.y + r16((o.y * r1) * wv.y)),
-                               r16(xr.z + r16((o.z * r1) * wv.z)), r16(xr.w + r16((o.w * r1) * wv.w)));
-        if (after_mlp) v = make_float4(r16(v.x * scal), r16(v.y * scal), r16(v.z * scal), r16(v.w * scal));
-        x1[k] = v;
-        if (blockIdx.x == 0) reinterpret_cast<float4*>(a.nrm_xout)[(size_t)w * RW4 + lane + 64 * k] = v;
+        const float4 o = ov[k], wt = w1[k], xr = xv[k];
+        x1[k] = make_float4(res1(o.x, xr.x, wt.x, r1), res1(o.y, xr.y, wt.y, r1), res1(o.z, xr.z, wt.z, r1),
+                            res1(o.w, xr.w, wt.w, r1));
+        if constexpr (XM == 1) reinterpret_cast<float4*>(XR)[u0 + 64 * k] = x1[k];
       }
-      float4 fin[PER];
-      if constexpr (XM == 1) {
+      if (blockIdx.x == 0)
 #pragma unroll
-        for (int k = 0; k < PER; ++k) fin[k] = x1[k];
-      } else {
-        float4 w2[PER];
-#pragma unroll
-        for (int k = 0; k < PER; ++k) w2[k] = w24[64 * k];
-        const float r2 = rms_row(x1);
+        for (int k = 0; k < PER; ++k) reinterpret_cast<float4*>(a.nrm_xout)[(size_t)wq * RW4 + u0 + 64 * k] = x1[k];
+      if constexpr (XM != 1) share_sumsq(x1, SSP[1], w);
+    }
+    if constexpr (XM != 1) {
+      lds_barrier();
+      if (live) {
+        const float r2 = 1.0f / sqrtf(row_mean<WPR>(SSP[1], 4 * WPR * wq, [&](int e) {
+                                        return res1(o_at(e), a.nrm_xin[(size_t)mr * H + e], a.nrm_w1[e], r1);
+                                      }) + 1e-6f);
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
-          const float4 tv = x1[k], wv = w2[k];
-          float4 v = make_float4((tv.x * r2) * wv.x, (tv.y * r2) * wv.y, (tv.z * r2) * wv.z, (tv.w * r2) * wv.w);
-          if (!after_mlp) v = make_float4(r16(v.x), r16(v.y), r16(v.z), r16(v.w));
-          fin[k] = v;
+          const float4 tv = x1[k], wt = w2[k];
+          reinterpret_cast<float4*>(XR)[u0 + 64 * k] =
+              make_float4(r16_if((tv.x * r2) * wt.x, !after_mlp), r16_if((tv.y * r2) * wt.y, !after_mlp),
+                          r16_if((tv.z * r2) * wt.z, !after_mlp), r16_if((tv.w * r2) * wt.w, !after_mlp));
         }
       }
-#pragma unroll
-      for (int k = 0; k < PER; ++k) reinterpret_cast<float4*>(XR)[lane + 64 * k] = fin[k];
     }
     if (tid < CG * G8 * 16) SWL[tid] = swr;
     __syncthreads();
@@ -598,31 +568,38 @@ int launch_gemv_a8(const GemvTArgs& a, hipStream_t st) {
   if (a.K != H) return 0;
   static bool raised = false;  // the norm variants stage more than 64 KB (gfx950: up to 160 KB on request)
   if (!raised) {
-    const void* fns[] = {reinterpret_cast<const void*>(&k_gemv_a8n<0, 4>), reinterpret_cast<const void*>(&k_gemv_a8n<0, 2>),
-                         reinterpret_cast<const void*>(&k_gemv_a8n<1, 1>),
-                         reinterpret_cast<const void*>(&k_gemv_a8n<0, 1>)};
-    for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 163840);
+    const void* fns[] = {
+        reinterpret_cast<const void*>(&k_gemv_a8n<0, 4, 1>), reinterpret_cast<const void*>(&k_gemv_a8n<0, 4, 2>),
+        reinterpret_cast<const void*>(&k_gemv_a8n<0, 2, 1>), reinterpret_cast<const void*>(&k_gemv_a8n<1, 1, 1>),
+        reinterpret_cast<const void*>(&k_gemv_a8n<1, 1, 2>), reinterpret_cast<const void*>(&k_gemv_a8n<0, 1, 1>),
+        reinterpret_cast<const void*>(&k_gemv_a8n<0, 1, 2>)};
+    for (const void* f : fns)  // (the rows' sums sit in static LDS)
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 163840 - 1024);
     raised = true;
   }
+  const bool two = a.M <= 4;  // waves per row of the prologue: the block's eight over its rows
   if (a.gateup) {
     if (a.epi_pli || a.mat[0].N != a.mat[1].N || a.mat[2].N) return 0;
     // 4 tiles a block (each block owns one 32-group of every row, quantised here for down)
     if (a8_gateup_quantises(a.mat[0].N)) {
       const int grid = a.mat[0].N / 32;
-      hipLaunchKernelGGL((k_gemv_a8n<0, 4>), dim3(grid), b, (a8n_lds<4>()), st, a);
+      if (two) hipLaunchKernelGGL((k_gemv_a8n<0, 4, 2>), dim3(grid), b, (a8n_lds<4>()), st, a);
+      else hipLaunchKernelGGL((k_gemv_a8n<0, 4, 1>), dim3(grid), b, (a8n_lds<4>()), st, a);
       return grid;
     }
     if (a.yq) return 0;  // (two tiles a block own half a group)
     const int grid = a.mat[0].N / 16;
-    hipLaunchKernelGGL((k_gemv_a8n<0, 2>), dim3(grid), b, (a8n_lds<2>()), st, a);
+    hipLaunchKernelGGL((k_gemv_a8n<0, 2, 1>), dim3(grid), b, (a8n_lds<2>()), st, a);
     return grid;
   }
   if (a.epi_pli) {
     if (a.nrm_mode != 3 || a.mat[1].N || a.mat[2].N) return 0;
-    hipLaunchKernelGGL((k_gemv_a8n<1, 1>), dim3(tiles), b, (a8n_lds<1>()), st, a);
+    if (two) hipLaunchKernelGGL((k_gemv_a8n<1, 1, 2>), dim3(tiles), b, (a8n_lds<1>()), st, a);
+    else hipLaunchKernelGGL((k_gemv_a8n<1, 1, 1>), dim3(tiles), b, (a8n_lds<1>()), st, a);
   } else {
     if (a.nrm_mode == 3) return 0;
-    hipLaunchKernelGGL((k_gemv_a8n<0, 1>), dim3(tiles), b, (a8n_lds<1>()), st, a);
+    if (two) hipLaunchKernelGGL((k_gemv_a8n<0, 1, 2>), dim3(tiles), b, (a8n_lds<1>()), st, a);
+    else hipLaunchKernelGGL((k_gemv_a8n<0, 1, 1>), dim3(tiles), b, (a8n_lds<1>()), st, a);
   }
   return tiles;
 }

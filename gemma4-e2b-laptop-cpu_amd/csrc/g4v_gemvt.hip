@@ -86,13 +86,11 @@ struct GemvTDev {
 
 // LDS: activations [MPL][G][8 + 1] float4 (staged; a pad float4 after each group spreads the
 // per-group accesses of the prologue over the banks), group sums [MPL][G], chain sums [MPL][8][64],
-// offsets [MPL][64], outputs of the gate/up epilogue [MPL][64]; the norm prologue adds its two
-// weight rows [2][H] and RMS factors [2][MPL]
-static size_t gemvt_lds(int mpl, int K, bool nrm, int tr, bool mrg) {
+// offsets [MPL][64], outputs of the gate/up epilogue [MPL][64]; the merge prologue adds its factors
+static size_t gemvt_lds(int mpl, int K, int tr, bool mrg) {
   const int G = K / 32;
   return (size_t)mpl * G * 9 * 16 + (size_t)mpl * G * 4 + (size_t)mpl * 8 * tr * 4 + (size_t)mpl * tr * 4 * 2 +
-         (mrg ? (size_t)mpl * NQ * (3 * MAXT + 1) * 4 : 0) +
-         (nrm ? (size_t)2 * H * 4 + (size_t)2 * mpl * 4 : 0);
+         (mrg ? (size_t)mpl * NQ * (3 * MAXT + 1) * 4 : 0);
 }
 
 // MRG: the merge prologue (GemvTArgs::mrg_po), NRM: the norm prologue (GemvTArgs::nrm_mode);
@@ -277,109 +275,81 @@ __global__ __launch_bounds__(TR * 8) void k_gemv_t(const float* __restrict__ pa,
     }
   } else if constexpr (NRM) {
     // E:1358-1361 (mode 1) / E:1375-1378 with E:1390-1404 (mode 2, the per-layer-embedding
-    // branch zero) for the block's rows.  Wave q forms row q in registers (6 float4 per lane)
-    // without block barriers: x1 = r16(xin + r16((r16(o) * r1) * w1)), then xa from x1 and r2,
-    // written to XL in plain order; XL is then permuted in place into the staged order, one
-    // thread per (row, group).
-    //
-    constexpr int RW4 = H / 4, PER = RW4 / 64;
-    static_assert(NT / 64 >= MPL, "a wave per activation row");
-    const int wq = threadIdx.x >> 6, ln = threadIdx.x & 63;
-    const bool rowwave = wq < MPL;            // uniform per wave
+    // branch zero) for the block's rows: x1 = r16(xin + r16((r16(o) * r1) * w1)), then xa from x1
+    // and r2, written to XL in plain order; XL is then permuted in place into the staged order, one
+    // thread per (row, group).  A row sits on WPR waves (PER float4 per lane), whose sums of
+    // squares meet in LDS (certified_mean); the barriers order LDS only, the weights stay in flight.
+    // With one wave a row and the reference's chains in it the prologue took 11.4k cycles of a
+    // 4-row gate / up block.
+    constexpr int NWV = NT / 64, WPR = NWV / MPL >= 3 ? 3 : (NWV / MPL == 2 ? 2 : 1);
+    constexpr int RW4 = H / 4, PER = RW4 / 64 / WPR;
+    static_assert(NWV >= MPL * WPR && PER * 64 * WPR == RW4, "whole waves per activation row");
+    __shared__ RmsShare SSP[2];
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), ln = threadIdx.x & 63;
+    const int wq = wv / WPR, u0 = ln + 64 * PER * (wv % WPR);  // the wave's row, its first float4
+    const bool rowwave = wq < MPL;             // uniform per wave
     const bool live = rowwave && m0 + wq < M;  // rows past M are staged as zeros
     const int mr = min(m0 + wq, M - 1);
-    const float4* o4 = reinterpret_cast<const float4*>(pa) + (size_t)mr * RW4 + ln;
-    const float4* x4 = reinterpret_cast<const float4*>(pb) + (size_t)mr * RW4 + ln;
-    const float4* w14 = reinterpret_cast<const float4*>(pc) + ln;
-    const float4* w24 = reinterpret_cast<const float4*>(pd) + ln;
-    float4 ov[PER], xv[PER];
+    const float4* o4 = reinterpret_cast<const float4*>(pa) + (size_t)mr * RW4 + u0;
+    const float4* x4 = reinterpret_cast<const float4*>(pb) + (size_t)mr * RW4 + u0;
+    const float4* w14 = reinterpret_cast<const float4*>(pc) + u0;
+    const float4* w24 = reinterpret_cast<const float4*>(pd) + u0;
+    float4 ov[PER], xv[PER], w1[PER], w2[PER];
     if (rowwave) {
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
         ov[k] = o4[64 * k];
         xv[k] = x4[64 * k];
+        w1[k] = w14[64 * k];
+        if constexpr (XM != 1) w2[k] = w24[64 * k];
       }
     }
     weights_after();
+    const bool after_mlp = nmode == 2;
+    const float scal = after_mlp ? a.nrm_scalar : 1.0f;  // (r16(v * 1) = v: no branch per element)
+    float4 x1[PER];
+    auto res1 = [&](float o, float xr, float w, float r1) { return r16(r16(xr + r16((o * r1) * w)) * scal); };
+    // the row's elements again, for the rare sum that needs the reference's order
+    auto o_at = [&](int e) { return r16(pa[(size_t)mr * H + e]); };
     if (rowwave) {
-      float4* XR = XL + (size_t)wq * G * 9;  // row wq, plain order (padded)
-      auto xl_at = [&](int k) -> float4& { const int u = ln + 64 * k; return XR[u + (u >> 3)]; };
-      // E:326-345: lane t of the reference's ss_avx2 sums x[16 s + t]^2 in double over s in
-      // order, and the 16 lane sums meet as a_l = (p_l + p_{l+4}) + (p_{l+8} + p_{l+12}),
-      // ss = (a_0 + a_2) + (a_1 + a_3).  The wave writes its row into its XL region chain-major
-      // (chain t at 100 t: the 96 values of one chain contiguous, rows of chains spread over the
-      // banks), lanes 0..15 run the 16 chains, and the sums meet through data-parallel moves.
-      float* CR = reinterpret_cast<float*>(XR);
-      auto rms_row = [&](const float4 (&v)[PER]) -> float {
-#pragma unroll
-        for (int k = 0; k < PER; ++k) {
-          const float f[4] = {v[k].x, v[k].y, v[k].z, v[k].w};
-#pragma unroll
-          for (int c = 0; c < 4; ++c) {
-            const int e = 4 * (ln + 64 * k) + c;  // element e: chain e % 16, step e / 16
-            CR[(e & 15) * 100 + (e >> 4)] = f[c];
-          }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        double part = 0;
-        if (ln < 16) {
-          const float4* ch = reinterpret_cast<const float4*>(CR + ln * 100);
-#pragma unroll
-          for (int i = 0; i < H / 64; ++i) {
-            const float4 q = ch[i];
-            const double d0 = (double)q.x, d1 = (double)q.y, d2 = (double)q.z, d3 = (double)q.w;
-            part = fma(d0, d0, part);
-            part = fma(d1, d1, part);
-            part = fma(d2, d2, part);
-            part = fma(d3, d3, part);
-          }
-        }
-        const double b2 = part + shl_d<4>(part);  // lane l: p_l + p_{l+4}
-        const double c2 = b2 + shl_d<8>(b2);      // lanes 0..3: a_l
-        const double d2 = c2 + shl_d<2>(c2);      // lanes 0, 1: a_0 + a_2, a_1 + a_3
-        const double e2 = d2 + shl_d<1>(d2);      // lane 0: ss
-        const uint64_t u = as_u64(e2);
-        const double ss = as_f64(((uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(u >> 32), 0) << 32) |
-                                 (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)u, 0));
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        return 1.0f / sqrtf((float)(ss / H) + 1e-6f);
-      };
-      const bool after_mlp = nmode == 2;
-      const float scal = a.nrm_scalar;
-      float4 w1[PER];
-#pragma unroll
-      for (int k = 0; k < PER; ++k) w1[k] = w14[64 * k];
-      float4 os[PER];
 #pragma unroll
       for (int k = 0; k < PER; ++k)
-        os[k] = keep4(live, make_float4(r16(ov[k].x), r16(ov[k].y), r16(ov[k].z), r16(ov[k].w)));
-      const float r1 = rms_row(os);
-      float4 x1[PER];
+        ov[k] = keep4(live, make_float4(r16(ov[k].x), r16(ov[k].y), r16(ov[k].z), r16(ov[k].w)));
+      share_sumsq(ov, SSP[0], wv);
+    }
+    lds_barrier();
+    float r1 = 0.f;
+    if (rowwave) {
+      r1 = 1.0f / sqrtf(row_mean<WPR>(SSP[0], 4 * WPR * wq, [&](int e) { return live ? o_at(e) : 0.f; }) + 1e-6f);
 #pragma unroll
       for (int k = 0; k < PER; ++k) {
-        const float4 o = os[k], w = w1[k], xr = xv[k];
-        float4 v = make_float4(r16(xr.x + r16((o.x * r1) * w.x)), r16(xr.y + r16((o.y * r1) * w.y)),
-                               r16(xr.z + r16((o.z * r1) * w.z)), r16(xr.w + r16((o.w * r1) * w.w)));
-        if (after_mlp) v = make_float4(r16(v.x * scal), r16(v.y * scal), r16(v.z * scal), r16(v.w * scal));
-        x1[k] = keep4(live, v);
-        if (t == 0 && live) reinterpret_cast<float4*>(a.nrm_xout)[(size_t)(m0 + wq) * RW4 + ln + 64 * k] = x1[k];
+        const float4 o = ov[k], w = w1[k], xr = xv[k];
+        x1[k] = keep4(live, make_float4(res1(o.x, xr.x, w.x, r1), res1(o.y, xr.y, w.y, r1), res1(o.z, xr.z, w.z, r1),
+                                        res1(o.w, xr.w, w.w, r1)));
       }
-      if constexpr (XM == 1) {  // (mode 3: x1 itself is the product's input)
+      if (t == 0 && live)
+#pragma unroll
+        for (int k = 0; k < PER; ++k)
+          reinterpret_cast<float4*>(a.nrm_xout)[(size_t)(m0 + wq) * RW4 + u0 + 64 * k] = x1[k];
+    }
+    float4* XR = XL + (size_t)min(wq, MPL - 1) * G * 9;  // row wq, plain order (padded)
+    auto xl_at = [&](int k) -> float4& { const int u = u0 + 64 * k; return XR[u + (u >> 3)]; };
+    if constexpr (XM == 1) {  // (mode 3: x1 itself is the product's input)
+      if (rowwave)
 #pragma unroll
         for (int k = 0; k < PER; ++k) xl_at(k) = x1[k];
-      } else {
-        float4 w2[PER];
-#pragma unroll
-        for (int k = 0; k < PER; ++k) w2[k] = w24[64 * k];
-        const float r2 = rms_row(x1);
+    } else {
+      if (rowwave) share_sumsq(x1, SSP[1], wv);
+      lds_barrier();
+      if (rowwave) {
+        const float r2 = 1.0f / sqrtf(row_mean<WPR>(SSP[1], 4 * WPR * wq, [&](int e) {
+                                        return live ? res1(o_at(e), pb[(size_t)mr * H + e], pc[e], r1) : 0.f;
+                                      }) + 1e-6f);
 #pragma unroll
         for (int k = 0; k < PER; ++k) {
           const float4 tv = x1[k], w = w2[k];
-          float4 v = make_float4((tv.x * r2) * w.x, (tv.y * r2) * w.y, (tv.z * r2) * w.z, (tv.w * r2) * w.w);
-          if (!after_mlp) v = make_float4(r16(v.x), r16(v.y), r16(v.z), r16(v.w));
-          xl_at(k) = v;
+          xl_at(k) = make_float4(r16_if((tv.x * r2) * w.x, !after_mlp), r16_if((tv.y * r2) * w.y, !after_mlp),
+                                 r16_if((tv.z * r2) * w.z, !after_mlp), r16_if((tv.w * r2) * w.w, !after_mlp));
         }
       }
     }
@@ -729,7 +699,7 @@ static GemvTLead gemvt_lead(const GemvTDev& d) {
 #define G4V_GEMVT_ARGS L.pa, L.pb, L.pc, L.pd, L.w0w, L.w0s, L.gx, L.tl, d
 template <int MPL, int TR>
 static void launch_mpl(const GemvTDev& d, hipStream_t st, int grid) {
-  const size_t lds = gemvt_lds(MPL, d.a.K, d.a.nrm_mode != 0, TR, d.a.mrg_po != nullptr);
+  const size_t lds = gemvt_lds(MPL, d.a.K, TR, d.a.mrg_po != nullptr);
   const dim3 g(grid), b(TR * 8);
   const int K = d.a.K;
   const GemvTLead L = gemvt_lead(d);

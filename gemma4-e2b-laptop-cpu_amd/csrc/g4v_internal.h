@@ -200,6 +200,111 @@ __device__ __forceinline__ void unroll_n(F& f) {
   unroll_impl(f, std::make_integer_sequence<int, N>{});
 }
 
+// ---- RMS sums (E:326-345): the reference adds 16 chains of squares in double, each in order, and
+// rounds ss / n to float.  The sum needs no order, and the 96-step chains (2.1-2.4k cycles on 16 lanes)
+// become a few steps on every lane, where one of two conditions holds; elsewhere the caller runs
+// the chains.
+//  - Any order of the same non-negative terms lies within (steps + steps') 2^-53 < 2^-44 of the
+//    reference's: if (float) gives one value over the mean's 2^-43 neighbourhood, it is the reference's.
+//  - Squares of bf16 values of exponent e are multiples of 2^(2 (e - 7)).  If the sum is below 2^52 such
+//    units of the row's smallest element, every partial sum in every order is exact.  (About one row in
+//    five of the synthetic stack sits on a rounding boundary with a sum of few bits: its values are
+//    coarse.  Those take the division; with this test the chains are left to rows of a wide range
+//    on a boundary.)
+__device__ __forceinline__ uint32_t rms_key(float v) { return (as_u32(v) & 0x7FFFFFFFu) - 1u; }  // 0: never the least
+__device__ __forceinline__ bool certified_mean(double ss, uint32_t least, int n, float& mean) {
+  const double d = ss * (1.0 / n);  // (2^-52 beside ss / n)
+  mean = (float)fma(d, -0x1p-43, d);
+  if (__builtin_expect(mean == (float)fma(d, 0x1p-43, d), 1)) return true;
+  const int e = max((int)((least + 1u) >> 23), 1) - 127;
+  if (!(ss < as_f64((uint64_t)(2 * (e - 7) + 52 + 1023) << 52))) return false;  // (infinities and NaN too)
+  mean = (float)(ss / n);
+  return true;
+}
+// the sums of v over each row of 16 lanes, on the row's lane 0
+__device__ __forceinline__ double row16_sum(double v) {
+  v = v + shl_d<8>(v);
+  v = v + shl_d<4>(v);
+  v = v + shl_d<2>(v);
+  return v + shl_d<1>(v);
+}
+// the least of each row of 16 lanes, on the row's lane 0
+template <int N>
+__device__ __forceinline__ uint32_t shl_min(uint32_t v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return min(v, (uint32_t)__builtin_amdgcn_update_dpp(-1, (int)v, 0x100 + N, 0xF, 0xF, false));
+#else
+  return v;
+#endif
+}
+__device__ __forceinline__ uint32_t row16_min(uint32_t v) { return shl_min<1>(shl_min<2>(shl_min<4>(shl_min<8>(v)))); }
+// the reference's order over n elements get(e), formed by one wave: lane t the chain of elements
+// 16 s + t, then a_l = (p_l + p_{l+4}) + (p_{l+8} + p_{l+12}), ss = (a_0 + a_2) + (a_1 + a_3)
+template <typename F>
+__device__ __forceinline__ double chain_sumsq(int n, F get) {
+  double part = 0;
+  for (int e = threadIdx.x & 15; e < n; e += 16) {
+    const double d = (double)get(e);
+    part = fma(d, d, part);
+  }
+  const double b2 = part + shl_d<4>(part);
+  const double c2 = b2 + shl_d<8>(b2);
+  const double d2 = c2 + shl_d<2>(c2);
+  const uint64_t u = as_u64(d2 + shl_d<1>(d2));
+#if defined(__HIP_DEVICE_COMPILE__)
+  return as_f64(((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(u >> 32)) << 32) |
+                (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)u));
+#else
+  return as_f64(u);
+#endif
+}
+// r16 (rnd) or v unchanged, without a branch
+__device__ __forceinline__ float r16_if(float v, bool rnd) {
+  const uint32_t u = as_u32(v), keep = rnd ? 0xFFFF0000u : 0xFFFFFFFFu;
+  return as_f32((u + ((0x7fffu + ((u >> 16) & 1u)) & ~keep)) & keep);
+}
+// A row of H bf16 values on WPR waves (PER float4 per lane): this wave's shares go to its four entries
+// in LDS, and after a block barrier row_mean reads the row's 4 WPR entries from e0 on.
+struct RmsShare {
+  double s[32];
+  uint32_t least[32];
+};
+template <int PER>
+__device__ __forceinline__ void share_sumsq(const float4 (&v)[PER], RmsShare& sh, int wave) {
+  double s = 0, t = 0;
+  uint32_t m = 0xFFFFFFFFu;
+#pragma unroll
+  for (int k = 0; k < PER; ++k) {
+    const double a = (double)v[k].x, b = (double)v[k].y, c = (double)v[k].z, d = (double)v[k].w;
+    s = fma(a, a, s);
+    t = fma(b, b, t);
+    s = fma(c, c, s);
+    t = fma(d, d, t);
+    m = min(min(m, rms_key(v[k].x)), rms_key(v[k].y));
+    m = min(min(m, rms_key(v[k].z)), rms_key(v[k].w));
+  }
+  s = row16_sum(s + t);
+  m = row16_min(m);
+  if ((threadIdx.x & 15) == 0) {
+    sh.s[4 * wave + ((threadIdx.x & 63) >> 4)] = s;
+    sh.least[4 * wave + ((threadIdx.x & 63) >> 4)] = m;
+  }
+}
+template <int WPR, typename F>
+__device__ __forceinline__ float row_mean(const RmsShare& sh, int e0, F get) {
+  double s = 0;
+  uint32_t m = 0xFFFFFFFFu;
+#pragma unroll
+  for (int i = 0; i < 4 * WPR; ++i) {
+    s += sh.s[e0 + i];
+    m = min(m, sh.least[e0 + i]);
+  }
+  float mean;
+  if (__builtin_expect(!certified_mean(s, m, H, mean), 0))  // uniform over the wave
+    mean = (float)(chain_sumsq(H, get) / H);
+  return mean;
+}
+
 // The 16-lane head order of a 256-wide head: element e = 16 tt + n at n * 16 + tt, so that lane n
 // of a row of 16 lanes reads its 16 elements (its sum-of-squares lane, score chain and RoPE
 // pairs, tt and tt + 8) as four 16-byte words.  Applied per head of 256 to wider rows.
@@ -297,6 +402,74 @@ struct GemvTArgs {
 // W4A8 (g4v_w4a8.hip): operand tiles of a matrix from its original bytes [N][K/2] and scales
 // [N][K/32] (N % 16 == 0): tw [N/16][K/128][64] uint4, ts [N/16][K/256][16] uint4
 void launch_tile_a8(const uint8_t* w, const uint16_t* s, uint4* tw, uint4* ts, int N, int K, hipStream_t st);
+// The quantised rows of a many-row W4A8 product (quant, engine/w4a8_avx2.h:30-42): q [rows][K] as bf16
+// with each 8-element slice in the order 0,2,4,6,1,3,5,7, its scales sx and corrections -136 sum(q),
+// [K / 32][ld].  Rows past the last are read by the matrix instructions and never stored: any value.
+struct A8Rows {
+  uint16_t* q;
+  float* sx;
+  float* corr;
+  int ld;
+};
+// q of x (RNE, as cvtps_epi32; 8-bit saturation; NaN gives 0) and its unsaturated integer
+__device__ __forceinline__ float a8_q(float x, float inv, float& sum) {
+  const int q = (int)__builtin_rintf(x * inv);
+  sum += (float)q;  // |q| <= 127 for finite x: the group's sum is exact
+  return (float)(q > 127 ? 127 : (q < -128 ? -128 : q));
+}
+// 8 consecutive values v of row m (values 8 i ..), four neighbouring lanes a group of 32
+__device__ __forceinline__ void a8_store8(const A8Rows& o, int m, int K, int i, const float (&v)[8]) {
+  float amax = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[k]));
+  amax = fmaxf(amax, dpp_f(amax, 2));
+  amax = fmaxf(amax, dpp_f(amax, 3));
+  const float sx = amax / 127.0f, inv = sx > 0.f ? 1.0f / sx : 0.0f;
+  float q[8], sum = 0.f;
+#pragma unroll
+  for (int k = 0; k < 8; ++k) q[k] = a8_q(v[k], inv, sum);
+  sum += dpp_f(sum, 2);
+  sum += dpp_f(sum, 3);
+  auto pair = [](float a, float b) { return (as_u32(a) >> 16) | (as_u32(b) & 0xFFFF0000u); };
+  *reinterpret_cast<uint4*>(o.q + (size_t)m * K + 8 * i) =
+      make_uint4(pair(q[0], q[2]), pair(q[4], q[6]), pair(q[1], q[3]), pair(q[5], q[7]));
+  if ((i & 3) == 0) {
+    o.sx[(size_t)(i >> 2) * o.ld + m] = sx;
+    o.corr[(size_t)(i >> 2) * o.ld + m] = -136.0f * sum;
+  }
+}
+// a row of H values x (LDS) of a block of 256 threads
+__device__ __forceinline__ void a8_store_row(const A8Rows& o, int m, const float* x) {
+  if (threadIdx.x < H / 8) {
+    const float4 a = *reinterpret_cast<const float4*>(x + 8 * threadIdx.x), b = *reinterpret_cast<const float4*>(x + 8 * threadIdx.x + 4);
+    const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+    a8_store8(o, m, H, threadIdx.x, v);
+  }
+}
+// max / sum over a row of 16 lanes, on every lane (quad permutes, then the mirrors of 8 and 16)
+template <int CTRL>
+__device__ __forceinline__ float dpp_any(float v) {
+#if defined(__HIP_DEVICE_COMPILE__)
+  return as_f32((uint32_t)__builtin_amdgcn_update_dpp(0, (int)as_u32(v), CTRL, 0xF, 0xF, false));
+#else
+  return v;
+#endif
+}
+__device__ __forceinline__ float row16_all_max(float v) {
+  v = fmaxf(v, dpp_any<0xB1>(v));
+  v = fmaxf(v, dpp_any<0x4E>(v));
+  v = fmaxf(v, dpp_any<0x141>(v));
+  return fmaxf(v, dpp_any<0x140>(v));
+}
+__device__ __forceinline__ float row16_all_sum(float v) {
+  v += dpp_any<0xB1>(v);
+  v += dpp_any<0x4E>(v);
+  v += dpp_any<0x141>(v);
+  return v + dpp_any<0x140>(v);
+}
+// the place of element e of a 32-group in the operand order
+__device__ __forceinline__ int a8_slot(int e) { return (e & ~7) + (e & 1) * 4 + ((e & 7) >> 1); }
+
 // quantised rows: xqb [Mpad][K] bf16 (MFMA operand order), sxt / corr [K/32][Mpad]; q / sx / sum
 // (optional, plain layouts [M][K], [M][K/32]) for the quant entry point
 void launch_w4a8_quant(const float* x, int M, int Mpad, int K, uint16_t* xqb, float* sxt, float* corr, int8_t* qo,

@@ -51,7 +51,42 @@ __device__ inline double block_sumsq(const float* x, int n, double* red16) {
 // E:345: r = 1 / sqrtf((float)(ss / n) + 1e-6)
 __device__ __forceinline__ float rms_inv(double ss, int n) { return 1.0f / sqrtf((float)(ss / n) + 1e-6f); }
 
-constexpr int ROW_THREADS = 256;
+// rms_inv(block_sumsq(x, N)) of N bf16 values, by a block of 256 threads, every one at work: the sum in
+// any order where it certifies the factor, else the reference's
+template <int N>
+__device__ inline float block_rms_inv(const float* x, double* red16) {
+  static_assert(N % 256 == 0, "whole rounds of the block");
+  __shared__ uint32_t least[16];
+  double s = 0;
+  uint32_t m = 0xFFFFFFFFu;
+#pragma unroll
+  for (int i = 0; i < N / 256; ++i) {
+    const float v = x[threadIdx.x + 256 * i];
+    const double d = (double)v;
+    s = fma(d, d, s);
+    m = min(m, rms_key(v));
+  }
+  s = row16_sum(s);
+  m = row16_min(m);
+  if ((threadIdx.x & 15) == 0) {
+    red16[threadIdx.x >> 4] = s;
+    least[threadIdx.x >> 4] = m;
+  }
+  __syncthreads();
+  double t = 0;
+  m = 0xFFFFFFFFu;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    t += red16[i];
+    m = min(m, least[i]);
+  }
+  __syncthreads();
+  float mean;
+  if (__builtin_expect(certified_mean(t, m, N, mean), 1)) return 1.0f / sqrtf(mean + 1e-6f);  // (uniform)
+  return rms_inv(block_sumsq(x, N, red16), N);
+}
+
+constexpr int ROW_THREADS = 256;  // (block_rms_inv counts on it)
 
 // per-layer pointers for the layer kernels
 struct LayerNorms {

@@ -63,7 +63,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_embed(const uint16_t* __restric
     x[(size_t)m * H + i] = v;
   }
   __syncthreads();
-  const float r = rms_inv(block_sumsq(xs, H, red), H);
+  const float r = block_rms_inv<H>(xs, red);
   for (int i = threadIdx.x; i < H; i += ROW_THREADS) ys[i] = (xs[i] * r) * in_ln[i];
   __syncthreads();
   write_staged(ys, H, xa + (size_t)m * H, xgs + (size_t)m * (H / 32));
@@ -91,7 +91,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_post_attn(const float* __restri
 #pragma unroll
   for (int k = 0; k < RPT; ++k) os[threadIdx.x + k * ROW_THREADS] = r16(ov[k]);
   __syncthreads();
-  const float r1 = rms_inv(block_sumsq(os, H, red), H);
+  const float r1 = block_rms_inv<H>(os, red);
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
     const int i = threadIdx.x + k * ROW_THREADS;
@@ -101,7 +101,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_post_attn(const float* __restri
     x[(size_t)m * H + i] = v;
   }
   __syncthreads();
-  const float r2 = rms_inv(block_sumsq(xs, H, red), H);
+  const float r2 = block_rms_inv<H>(xs, red);
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
     const int i = threadIdx.x + k * ROW_THREADS;
@@ -136,7 +136,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_post_ff(const float* __restrict
 #pragma unroll
   for (int k = 0; k < RPT; ++k) os[threadIdx.x + k * ROW_THREADS] = r16(ov[k]);
   __syncthreads();
-  const float r1 = rms_inv(block_sumsq(os, H, red), H);
+  const float r1 = block_rms_inv<H>(os, red);
 #pragma unroll
   for (int k = 0; k < RPT; ++k) {
     const int i = threadIdx.x + k * ROW_THREADS;
@@ -147,7 +147,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_post_ff(const float* __restrict
     x[(size_t)m * H + i] = v;
   }
   __syncthreads();
-  const float r2 = rms_inv(block_sumsq(xs, H, red), H);
+  const float r2 = block_rms_inv<H>(xs, red);
   if (next_in_ln) {
 #pragma unroll
     for (int k = 0; k < RPT; ++k) {

@@ -67,8 +67,14 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_embed(const uint16_t* __rest
     x[(size_t)m * H + i] = v;
   }
   __syncthreads();
-  const float r = rms_inv(block_sumsq(xs, H, red), H);
-  for (int i = threadIdx.x; i < H; i += ROW_THREADS) a[(size_t)m * H + i] = (xs[i] * r) * in_ln[i];
+  const float r = block_rms_inv<H>(xs, red);
+  if (!aq.q) {  // (uniform)
+    for (int i = threadIdx.x; i < H; i += ROW_THREADS) a[(size_t)m * H + i] = (xs[i] * r) * in_ln[i];
+    return;
+  }
+  for (int i = threadIdx.x; i < H; i += ROW_THREADS) xs[i] = (xs[i] * r) * in_ln[i];
+  __syncthreads();
+  a8_store_row(aq, m, xs);
 }
 
 // E:1291-1303 / 1307-1324 for one row: the 8 query heads and k normed with their weights, v
@@ -523,15 +529,21 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_attn(const float* __res
   const int m = blockIdx.x;
   for (int i = threadIdx.x; i < H; i += ROW_THREADS) os[i] = r16(o[(size_t)m * H + i]);
   __syncthreads();
-  const float r1 = rms_inv(block_sumsq(os, H, red), H);
+  const float r1 = block_rms_inv<H>(os, red);
   for (int i = threadIdx.x; i < H; i += ROW_THREADS) {
     const float v = r16(x[(size_t)m * H + i] + r16((os[i] * r1) * w1[i]));
     xs[i] = v;
     x[(size_t)m * H + i] = v;
   }
   __syncthreads();
-  const float r2 = rms_inv(block_sumsq(xs, H, red), H);
-  for (int i = threadIdx.x; i < H; i += ROW_THREADS) a[(size_t)m * H + i] = r16((xs[i] * r2) * w2[i]);
+  const float r2 = block_rms_inv<H>(xs, red);
+  if (!aq.q) {  // (uniform)
+    for (int i = threadIdx.x; i < H; i += ROW_THREADS) a[(size_t)m * H + i] = r16((xs[i] * r2) * w2[i]);
+    return;
+  }
+  for (int i = threadIdx.x; i < H; i += ROW_THREADS) xs[i] = r16((xs[i] * r2) * w2[i]);
+  __syncthreads();
+  a8_store_row(aq, m, xs);
 }
 
 // E:1369-1370: act = r16(r16(gelu8(r16 g)) * r16 u)
@@ -557,7 +569,7 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_ff(const float* __restr
   const int m = blockIdx.x;
   for (int i = threadIdx.x; i < H; i += ROW_THREADS) os[i] = r16(o[(size_t)m * H + i]);
   __syncthreads();
-  const float r1 = rms_inv(block_sumsq(os, H, red), H);
+  const float r1 = block_rms_inv<H>(os, red);
   for (int i = threadIdx.x; i < H; i += ROW_THREADS) {
     float v = r16(x[(size_t)m * H + i] + r16((os[i] * r1) * w1[i]));
     v = r16(v * scalar);
@@ -566,8 +578,12 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_ff(const float* __restr
   }
   if (!next_in_ln && (hrow < 0 || m < hrow)) return;  // uniform
   __syncthreads();
-  const float r2 = rms_inv(block_sumsq(xs, H, red), H);
-  if (next_in_ln) {
+  const float r2 = block_rms_inv<H>(xs, red);
+  if (next_in_ln && aq.q) {
+    for (int i = threadIdx.x; i < H; i += ROW_THREADS) xs[i] = (xs[i] * r2) * next_in_ln[i];
+    __syncthreads();
+    a8_store_row(aq, m, xs);
+  } else if (next_in_ln) {
     for (int i = threadIdx.x; i < H; i += ROW_THREADS) a[(size_t)m * H + i] = (xs[i] * r2) * next_in_ln[i];
   } else {
     float* hr = h + (size_t)(m - hrow) * H;
@@ -597,7 +613,7 @@ __global__ __launch_bounds__(256) void k_gm_ple(const float* __restrict__ pr, co
   const float s1 = 1.0f / sqrtf((float)H);
   xs[i] = r16(pr[base + i] * s1);
   __syncthreads();
-  const float r = rms_inv(block_sumsq(xs, PD, red), PD);
+  const float r = block_rms_inv<PD>(xs, red);
   const float pj = (xs[i] * r) * plnorm[i];
   const float pev = r16(bf2f(ple[(size_t)toks[m] * NLG * PD + (size_t)l * PD + i]) * 16.0f);
   pli[base + i] = (pj + pev) * 0.70710678118f;

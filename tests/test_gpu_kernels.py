@@ -130,6 +130,37 @@ def test_norm_gemm_bit_exact(orc, dev, mode, kind, M, rpb, tr):
     assert same(y, ye), first_diff(y, ye)
 
 
+def _tie_row(rng, tail):
+    """1536 values whose mean square lies on (tail 0) or 2^-44-scale steps beside the middle of two
+    floats: 1 + 2^-24 + tail 2^-44 / 1536, where only the sum in the reference's order rounds as it
+    does (and no neighbourhood of the sum settles it)"""
+    v = np.ones(1536, np.float32)
+    v[:6], v[6:8] = 2.0 ** -8, 2.0
+    v[8:8 + tail] = 2.0 ** -22              # three ones become small squares ...
+    v[100:100 + tail // 3] = 2.0            # ... and one a two, so the whole squares still add up to 1536
+    return rng.permutation(v)
+
+
+@pytest.mark.parametrize("mode,M,rpb,tr", [(1, 4, 4, 64), (1, 7, 2, 64), (2, 5, 3, 64), (1, 3, 1, 64), (2, 1, 1, 32),
+                                           (1, 6, 2, 32), (1, 8, 4, 32)])
+def test_norm_gemm_ties(orc, dev, mode, M, rpb, tr):
+    """rows whose mean square sits on a rounding boundary, in either RMS: the factor needs the
+    reference's order of summation (every wave layout of the prologue)"""
+    rng = np.random.default_rng(100 * mode + 10 * M + rpb)
+    seed = 900 + M
+    W, S = _w4(orc, seed, 256, 1536)
+    o = np.stack([_tie_row(rng, 3 * (m % 3)) for m in range(M)])
+    xin = np.stack([_tie_row(rng, 3 * ((m + 1) % 3)) for m in range(M)])
+    o[M // 2:] = 0  # x1 = xin (halved in mode 2): the second sum on the boundary
+    w1 = orc.r16(0.5 + orc.normal_f32(orc.stream(seed, 7), 1536) ** 2 / 4)
+    w2 = orc.r16(0.5 + orc.normal_f32(orc.stream(seed, 8), 1536) ** 2 / 4)
+    note(f"norm gemm ties mode={mode} M={M} rows/block={rpb} tile={tr}")
+    y, x1 = dev.w4g32_norm(dev.w4_upload(W, S), mode, o, xin, w1, w2, 0.5, rpb, tr)
+    ye, x1e = _norm_expected(orc, W, S, mode, o, xin, w1, w2, 0.5)
+    assert same(x1, x1e), first_diff(x1, x1e)
+    assert same(y, ye), first_diff(y, ye)
+
+
 def _attn_case(orc, ctx, M, T, window, tree, seed, hd=256):
     nh = 8
     Kc = orc.normal_bf16(orc.stream(seed, 1), (ctx + 8) * hd)
