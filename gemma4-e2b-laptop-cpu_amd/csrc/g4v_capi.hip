@@ -2844,6 +2844,22 @@ extern "C" int g4v_drafter_synth(g4v_ctx* c, uint64_t seed) {
     launch_gen_bf16_normal(b.as<uint16_t>(), n, rng_stream(seed, tag), scale, st);
     return 0;
   };
+// the drafter's matrices, as generated or loaded, into the layout its products read
+static void dr_chains(g4v_ctx* c) {
+  hipStream_t st = c->st;
+  launch_b16_chains(c->dr_pre.as<uint16_t>(), DR_H, 2 * H, st);
+  launch_b16_chains(c->dr_post.as<uint16_t>(), H, DR_H, st);
+  launch_b16_chains(c->dr_cent.as<uint16_t>(), c->V / 128, DR_H, st);
+  launch_b16_chains(c->dr_emb.as<uint16_t>(), c->V, DR_H, st);
+  for (int l = 0; l < 4; ++l) {
+    launch_b16_chains(c->dr_q[l].as<uint16_t>(), DR_Q * c->dr_hd[l], DR_H, st);
+    launch_b16_chains(c->dr_o[l].as<uint16_t>(), DR_H, DR_Q * c->dr_hd[l], st);
+    launch_b16_chains(c->dr_g[l].as<uint16_t>(), DR_F, DR_H, st);
+    launch_b16_chains(c->dr_u[l].as<uint16_t>(), DR_F, DR_H, st);
+    launch_b16_chains(c->dr_d[l].as<uint16_t>(), DR_H, DR_F, st);
+  }
+}
+
   int r;
   if ((r = gen(c->dr_pre, (size_t)DR_H * 2 * H, 5000, 0.02f))) return r;
   for (int l = 0; l < 4; ++l) {
@@ -2904,6 +2920,7 @@ extern "C" int g4v_drafter_load(g4v_ctx* c, const g4v_drafter_tensors* t) {
   for (int l = 0; l < 4; ++l) {
     ARGCHK(t->q[l] && t->o[l] && t->gate[l] && t->up[l] && t->down[l], "drafter_load: null tensor");
     for (int k = 0; k < 5; ++k) ARGCHK(t->nv[l][k], "drafter_load: null norm");
+  dr_chains(c);
   }
   for (long long i = 0; i < V; ++i)
     ARGCHK(t->order[i] >= 0 && t->order[i] < V, "drafter_load: token ordering outside the vocabulary");
@@ -2973,6 +2990,8 @@ static void enqueue_draft(g4v_ctx* c, int k, int nsplit) {
       L.E = c->E.as<uint16_t>(), L.tok = d.tok + j;
       launch_b16(L, st);
     }
+  dr_chains(c);
+  HIPCHK(hipGetLastError());
     for (int l = 0; l < 4; ++l) {
       const bool sliding = l < 3;
       const int ty = sliding ? 0 : 1, ol = sliding ? 13 : 14, hd = c->dr_hd[l];  // E:1540

@@ -203,6 +203,8 @@ void launch_dr_qnorm(float* q, const float* qn, const float* cs, const float* sn
 // a chain's inputs: in = {tok, P, hrow, _, h[1536]}; hin = h (hrow < 0) or hbase row hrow;
 // tok[0] = tok; geo[2 j + s] = the attention geometry of step j on sliding (s = 0) / global layers
 void launch_dr_setup(const int* in, const float* hbase, float* hin, int* tok, AttnGeom* geo, int k, int T,
+// a bf16 matrix [rows][K] into the chain-major rows launch_b16 reads, in place (K % 128 == 0, K <= 3072)
+void launch_b16_chains(uint16_t* W, int rows, int K, hipStream_t st);
                      hipStream_t st);
 void launch_dr_rank(const float* score, int C, int* top, hipStream_t st);
 void launch_dr_best(const float* cs, const int* top, const int* order, int nc, int* tok, int* sec, float* gap,

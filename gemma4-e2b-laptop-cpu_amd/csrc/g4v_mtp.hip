@@ -30,12 +30,12 @@ enum { B16_PLAIN = 0, B16_RMS = 1, B16_RMS_R16 = 2, B16_COMB = 3, B16_RES0 = 4, 
 enum { B16_STORE = 0, B16_R16 = 1, B16_GATEUP = 2 };                  // output epilogue
 
 struct B16Args {
-  const uint16_t* W;   // [rows][K] bf16
+  const uint16_t* W;   // [rows][K] bf16, chain-major
   const uint16_t* W2;  // B16_GATEUP: the up matrix
   const int* rows;     // row of output n, or null: row n (or, with top: order[top[n / 128] 128 + n % 128])
   const int* top;
   const int* order;
-  int N, K;
+  int N;
   const float* x;      // input [K], or the prologue's source
   const float* nw;     // norm weights (B16_RMS*)
   const uint16_t* E;   // B16_COMB: token embedding [V][1536] ...
@@ -48,76 +48,100 @@ struct B16Args {
   float scalar;        // RES1*: the layer scalar
 };
 
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
+
+// [rows][K] to chain-major, a block per row, in place
 constexpr int B16_MAXK = 3072;
+__global__ __launch_bounds__(256) void k_b16_chains(uint16_t* __restrict__ W, int K) {
+  __shared__ uint16_t row[B16_MAXK];
+  uint16_t* w = W + (size_t)blockIdx.x * K;
+  for (int i = threadIdx.x; i < K; i += 256) row[i] = w[i];
+  __syncthreads();
+  for (int i = threadIdx.x; i < K; i += 256) w[(i & 15) * (K / 16) + (i >> 4)] = row[i];
+}
 constexpr int DR_MAXC = 4096;  // centroids
 
-template <int PRO, int EPI>
+// Weights are kept chain-major (launch_b16_chains): row r's element 16 s + l at r K + l (K / 16) + s, so
+// lane l's chain is K / 16 consecutive values, 16-byte loads that are all issued before the prologue
+// (with 2-byte loads after it a product took 5.0 us, with its K of 256 or 2048 against a launch of
+// 4.5).  The input is staged the same way, a pad of 4 floats per chain.
+template <int PRO, int EPI, int KT>
 __global__ __launch_bounds__(256) void k_b16(B16Args a) {
-  __shared__ __align__(16) float xs[B16_MAXK];
+  constexpr int CH = KT / 16, CP = CH + 4, NV = CH / 8;  // values of a chain, its LDS stride, its 16-byte words
+  constexpr bool NORM = PRO == B16_RMS || PRO == B16_RMS_R16 || PRO >= B16_RES0;
+  static_assert(!NORM || KT == 256, "a thread per element of a norm's input");
+  __shared__ __align__(16) float xp[16 * CP];
+  __shared__ float xs[NORM ? KT : 1];
   __shared__ double red[16];
-  const int K = a.K;
-  if (PRO == B16_COMB) {
-    const int tk = *a.tok;
-    const float sqh = sqrtf((float)H);
-    for (int i = threadIdx.x; i < H; i += 256) {
-      xs[i] = r16(bf2f(a.E[(size_t)tk * H + i]) * sqh);  // E:1537
-      xs[H + i] = a.x[i];
-    }
-  } else if (PRO >= B16_RES0) {  // K == 256 == blockDim.x: thread i owns element i
-    const int i = threadIdx.x;
-    xs[i] = r16(a.yin[i]);
-    __syncthreads();
-    const float r1 = rms_inv(block_sumsq(xs, 256, red), 256);
-    float v = r16(a.x[i] + r16((xs[i] * r1) * a.w1[i]));
-    if (PRO != B16_RES0) v = r16(v * a.scalar);
-    if (a.dxout && blockIdx.x == 0) a.dxout[i] = v;
-    __syncthreads();  // every thread has read xs
-    xs[i] = v;
-  } else {
-    for (int i = threadIdx.x; i < K; i += 256) xs[i] = a.x[i];
-  }
-  __syncthreads();
-  if (PRO == B16_RMS || PRO == B16_RMS_R16 || PRO >= B16_RES0) {  // E:345: (x * r) * w
-    const bool rnd = PRO == B16_RMS_R16 || PRO == B16_RES0 || PRO == B16_RES1_R16;
-    const float r = rms_inv(block_sumsq(xs, K, red), K);
-    for (int i = threadIdx.x; i < K; i += 256) {
-      const float v = (xs[i] * r) * a.nw[i];
-      xs[i] = rnd ? r16(v) : v;
-    }
-    __syncthreads();
-  }
-  if (a.xout && blockIdx.x == 0)
-    for (int i = threadIdx.x; i < K; i += 256) a.xout[i] = xs[i];
   const int n = blockIdx.x * 16 + (threadIdx.x >> 4), l = threadIdx.x & 15;
   const bool live = n < a.N;
   const size_t row = !live ? 0
                      : a.rows ? (size_t)a.rows[n]
                      : a.top  ? (size_t)a.order[(size_t)a.top[n >> 7] * 128 + (n & 127)]
                               : (size_t)n;
-  const uint16_t* w = a.W + row * K + l;
-  const uint16_t* w2 = EPI == B16_GATEUP ? a.W2 + row * K + l : nullptr;
-  float acc = 0.f, acc2 = 0.f;
-  if (live) {
-    // chain l: elements l, 16 + l, ... in order; the weights of 32 steps are loaded ahead of
-    // their FMAs (K is a multiple of 512 here or the tail loop takes the rest)
-    int k = 0;
-    for (; k + 512 <= K; k += 512) {
-      uint16_t wb[32], wb2[32];
+  u32x4_t wv[NV], wv2[EPI == B16_GATEUP ? NV : 1];
+  const u32x4_t* w4 = reinterpret_cast<const u32x4_t*>(a.W + row * KT + l * CH);
 #pragma unroll
-      for (int u = 0; u < 32; ++u) {
-        wb[u] = w[k + 16 * u];
-        if (EPI == B16_GATEUP) wb2[u] = w2[k + 16 * u];
-      }
+  for (int v = 0; v < NV; ++v) wv[v] = w4[v];
+  if constexpr (EPI == B16_GATEUP) {
+    const u32x4_t* u4 = reinterpret_cast<const u32x4_t*>(a.W2 + row * KT + l * CH);
 #pragma unroll
-      for (int u = 0; u < 32; ++u) {
-        acc = fmaf(bf2f(wb[u]), xs[k + 16 * u + l], acc);
-        if (EPI == B16_GATEUP) acc2 = fmaf(bf2f(wb2[u]), xs[k + 16 * u + l], acc2);
-      }
+    for (int v = 0; v < NV; ++v) wv2[v] = u4[v];
+  }
+  auto put = [&](int i, float v) { xp[(i & 15) * CP + (i >> 4)] = v; };
+  const int i = threadIdx.x;
+  if constexpr (PRO == B16_COMB) {
+    const int tk = *a.tok;
+    const float sqh = sqrtf((float)H);
+    for (int e = i; e < H; e += 256) {
+      put(e, r16(bf2f(a.E[(size_t)tk * H + e]) * sqh));  // E:1537
+      put(H + e, a.x[e]);
     }
-#pragma unroll 8
-    for (; k < K; k += 16) {
-      acc = fmaf(bf2f(w[k]), xs[k + l], acc);
-      if (EPI == B16_GATEUP) acc2 = fmaf(bf2f(w2[k]), xs[k + l], acc2);
+  } else if constexpr (!NORM) {
+    for (int e = i; e < KT; e += 256) {
+      const float v = a.x[e];
+      put(e, v);
+      if (a.xout && blockIdx.x == 0) a.xout[e] = v;
+    }
+  } else {  // thread i owns element i
+    const float nw = a.nw[i];
+    float v = a.x[i];
+    if constexpr (PRO >= B16_RES0) {
+      const float w1 = a.w1[i], o = r16(a.yin[i]);
+      xs[i] = o;
+      __syncthreads();
+      const float r1 = rms_inv(block_sumsq(xs, 256, red), 256);
+      v = r16(v + r16((o * r1) * w1));
+      if (PRO != B16_RES0) v = r16(v * a.scalar);
+      if (a.dxout && blockIdx.x == 0) a.dxout[i] = v;
+      __syncthreads();  // every thread is done with xs
+    }
+    xs[i] = v;
+    __syncthreads();
+    const bool rnd = PRO == B16_RMS_R16 || PRO == B16_RES0 || PRO == B16_RES1_R16;
+    const float r = rms_inv(block_sumsq(xs, 256, red), 256);
+    const float y = (v * r) * nw;  // E:345: (x * r) * w
+    v = rnd ? r16(y) : y;
+    put(i, v);
+    if (a.xout && blockIdx.x == 0) a.xout[i] = v;
+  }
+  __syncthreads();
+  float acc = 0.f, acc2 = 0.f;
+  if (live) {  // chain l: elements l, 16 + l, ... in order
+    const float4* x4 = reinterpret_cast<const float4*>(xp + l * CP);
+#pragma unroll
+    for (int v = 0; v < NV; ++v) {
+      const float4 x0 = x4[2 * v], x1 = x4[2 * v + 1];
+      const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const uint32_t u = wv[v][k >> 1];
+        acc = fmaf(as_f32((k & 1) ? (u & 0xFFFF0000u) : (u << 16)), x[k], acc);
+        if constexpr (EPI == B16_GATEUP) {
+          const uint32_t u2 = wv2[v][k >> 1];
+          acc2 = fmaf(as_f32((k & 1) ? (u2 & 0xFFFF0000u) : (u2 << 16)), x[k], acc2);
+        }
+      }
     }
   }
   // lanes 0..7 of each 16-lane group: v_l = a_l + b_l, then ((v0+v4)+(v1+v5))+((v2+v6)+(v3+v7))
@@ -211,18 +235,19 @@ __global__ __launch_bounds__(256) void k_dr_setup(const int* __restrict__ in, co
 }
 
 // E:1554-1555 top-32 centroids (descending, equal scores in index order): centroid c's place is
-// the count of scores above it plus the equal scores before it.  A block ranks 64 centroids;
-// its 4 waves count over the four quarters of the scores (LDS, 4 scores per read).
+// the count of scores above it plus the equal scores before it.  A block ranks 16 centroids, 16
+// threads each counting over every 16th group of 4 scores (64 a block, a quarter of the scores a
+// thread, took 22.4 us for 2,048 centroids on 32 blocks).
 __global__ __launch_bounds__(256) void k_dr_rank(const float* __restrict__ score, int C, int* __restrict__ top) {
   __shared__ __align__(16) float s[DR_MAXC];
-  __shared__ int part[4][64];
+  __shared__ int part[16][16];
   for (int j = threadIdx.x; j < C; j += 256) s[j] = score[j];
   __syncthreads();
-  const int cl = threadIdx.x & 63, q = threadIdx.x >> 6, c = blockIdx.x * 64 + cl;
-  const float v = c < C ? s[c] : 0.f;
-  const int j0 = q * (C / 4), j1 = q == 3 ? C : j0 + C / 4;  // C % 4 == 0
+  const int cl = threadIdx.x & 15, q = threadIdx.x >> 4, c = blockIdx.x * 16 + cl;  // C % 16 == 0
+  const float v = s[c];
   int rank = 0;
-  for (int j = j0; j < j1; j += 4) {
+#pragma unroll 4
+  for (int j = 4 * q; j < C; j += 64) {
     const float4 u = *reinterpret_cast<const float4*>(&s[j]);
     rank += (u.x > v) || (u.x == v && j < c);
     rank += (u.y > v) || (u.y == v && j + 1 < c);
@@ -231,8 +256,10 @@ __global__ __launch_bounds__(256) void k_dr_rank(const float* __restrict__ score
   }
   part[q][cl] = rank;
   __syncthreads();
-  if (q == 0 && c < C) {
-    rank = (part[0][cl] + part[1][cl]) + (part[2][cl] + part[3][cl]);
+  if (q == 0) {
+    rank = 0;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) rank += part[k][cl];
     if (rank < 32) top[rank] = c;
   }
 }
@@ -298,22 +325,29 @@ __global__ __launch_bounds__(1024) void k_dr_best(const float* __restrict__ cs, 
 }  // namespace
 
 void launch_b16(const B16Launch& L, hipStream_t st) {
-  B16Args a{L.W, L.W2, L.rows, L.top, L.order, L.N, L.K, L.x, L.nw, L.E, L.tok, L.y, L.xout, L.yin, L.w1, L.dxout,
+  B16Args a{L.W, L.W2, L.rows, L.top, L.order, L.N, L.x, L.nw, L.E, L.tok, L.y, L.xout, L.yin, L.w1, L.dxout,
             L.scalar};
   const dim3 grid((L.N + 15) / 16), block(256);
-#define G4V_B16(P, E) hipLaunchKernelGGL((k_b16<P, E>), grid, block, 0, st, a)
-  switch (L.pro * 3 + L.epi) {
-    case B16_PLAIN * 3 + B16_STORE: G4V_B16(B16_PLAIN, B16_STORE); break;
-    case B16_PLAIN * 3 + B16_R16: G4V_B16(B16_PLAIN, B16_R16); break;
-    case B16_RMS * 3 + B16_STORE: G4V_B16(B16_RMS, B16_STORE); break;
-    case B16_COMB * 3 + B16_R16: G4V_B16(B16_COMB, B16_R16); break;
-    case B16_RES0 * 3 + B16_GATEUP: G4V_B16(B16_RES0, B16_GATEUP); break;
-    case B16_RES1 * 3 + B16_STORE: G4V_B16(B16_RES1, B16_STORE); break;
-    case B16_RES1_R16 * 3 + B16_STORE: G4V_B16(B16_RES1_R16, B16_STORE); break;
-    case B16_RES1_R16 * 3 + B16_R16: G4V_B16(B16_RES1_R16, B16_R16); break;
+#define G4V_B16(P, E, K) hipLaunchKernelGGL((k_b16<P, E, K>), grid, block, 0, st, a)
+  switch (L.pro * 3 + L.epi) {  // the drafter's products: K 256, o's 4 hd, down's 2048, the pre-projection's 3072
+    case B16_PLAIN * 3 + B16_STORE:
+      if (L.K == 256) G4V_B16(B16_PLAIN, B16_STORE, 256);
+      else if (L.K == 1024) G4V_B16(B16_PLAIN, B16_STORE, 1024);
+      else if (L.K == 2048) G4V_B16(B16_PLAIN, B16_STORE, 2048);
+      break;
+    case B16_RMS * 3 + B16_STORE: G4V_B16(B16_RMS, B16_STORE, 256); break;
+    case B16_COMB * 3 + B16_R16: G4V_B16(B16_COMB, B16_R16, 2 * H); break;
+    case B16_RES0 * 3 + B16_GATEUP: G4V_B16(B16_RES0, B16_GATEUP, 256); break;
+    case B16_RES1 * 3 + B16_STORE: G4V_B16(B16_RES1, B16_STORE, 256); break;
+    case B16_RES1_R16 * 3 + B16_STORE: G4V_B16(B16_RES1_R16, B16_STORE, 256); break;
+    case B16_RES1_R16 * 3 + B16_R16: G4V_B16(B16_RES1_R16, B16_R16, 256); break;
     default: break;  // not used by the drafter
   }
 #undef G4V_B16
+}
+
+void launch_b16_chains(uint16_t* W, int rows, int K, hipStream_t st) {
+  hipLaunchKernelGGL(k_b16_chains, dim3(rows), dim3(256), 0, st, W, K);
 }
 
 void launch_dr_qnorm(float* q, const float* qn, const float* cs, const float* sn, const int* Pp, int j, int hd,
@@ -326,7 +360,7 @@ void launch_dr_setup(const int* in, const float* hbase, float* hin, int* tok, At
   hipLaunchKernelGGL(k_dr_setup, dim3(1), dim3(256), 0, st, in, hbase, hin, tok, geo, k, T);
 }
 void launch_dr_rank(const float* score, int C, int* top, hipStream_t st) {
-  hipLaunchKernelGGL(k_dr_rank, dim3((C + 63) / 64), dim3(256), 0, st, score, C, top);
+  hipLaunchKernelGGL(k_dr_rank, dim3(C / 16), dim3(256), 0, st, score, C, top);
 }
 void launch_dr_best(const float* cs, const int* top, const int* order, int nc, int* tok, int* sec, float* gap,
                     hipStream_t st) {
