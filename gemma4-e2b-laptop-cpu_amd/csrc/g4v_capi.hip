@@ -142,6 +142,7 @@ struct g4v_ctx {
   bool gm_plready = false;
   // prefill rows (plain [row][K] layouts), quantised activations, attention score scratch
   DBuf pfx, pfa, pfq, pfk, pfv, pfatt, pfo, pfg, pfu, pfact, pfxq, pfsx, pfcorr, pfs, pftok, pfh;
+  DBuf pfxq2, pfsx2, pfcorr2;  // the quantised activation, written while pfxq is the gate / up products' input
   int pf_rows = 0, pf_I = 0;  // rows and FFN width the buffers were sized for
   size_t pf_sfl = 0;
   // MTP drafter: tensors, then scratch of a chain (dx, da, y, q, att, act, dh, two hidden
@@ -1757,9 +1758,16 @@ static int verify_pass(g4v_ctx* c, const int* toks, int na, int nb, int pos0, in
 // ---------------------------------------------------------------------------------------
 // prefill
 // ---------------------------------------------------------------------------------------
+// the quantised rows of a W4A8 pass of M rows: set 0 a product's input, set 1 the MLP's activation
+static A8Rows pf_rows(g4v_ctx* c, int M, int set) {
+  return set ? A8Rows{c->pfxq2.as<uint16_t>(), c->pfsx2.as<float>(), c->pfcorr2.as<float>(), w4a8_mpad(M)}
+             : A8Rows{c->pfxq.as<uint16_t>(), c->pfsx.as<float>(), c->pfcorr.as<float>(), w4a8_mpad(M)};
+}
+// what the kernel before a product gets: those rows where the product is a many-row W4A8 one
+static A8Rows pf_out(g4v_ctx* c, int M, bool i8) { return i8 && M > 8 ? pf_rows(c, M, 0) : A8Rows{}; }
 // a linear layer of a prefill segment: lin_multi / lin1 (E:310-317) take W4A8 when the block has
-// M >= 2 rows (G_I8_ACTIVE during prefill), else the exact-float GEMV.  quant = false reuses the
-// quantised rows of the previous call (same x).
+// M >= 2 rows (G_I8_ACTIVE during prefill), else the exact-float GEMV.  quant = false: with more than 8
+// rows, x's quantised rows were left in `set` by the kernel before.
 //
 // the exact-float products of more than MAXM rows over the W4A8 operand tiles (the matrix-core
 // GEMM, g4v_gemmx.hip; every model matrix has N % 16 == 0); false: at most MAXM rows, the GEMV's.  The
@@ -1784,13 +1792,11 @@ static bool pf_exact(g4v_ctx* c, int n, const Mat* const* m, const float* x, int
   return true;
 }
 
-static void pf_lin(g4v_ctx* c, const Mat& m, const float* x, int M, float* y, bool i8, bool quant) {
+static void pf_lin(g4v_ctx* c, const Mat& m, const float* x, int M, float* y, bool i8, bool quant, int set = 0) {
   if (i8) {
-    if (quant)
-      launch_w4a8_quant(x, M, w4a8_mpad(M), m.K, c->pfxq.as<uint16_t>(), c->pfsx.as<float>(), c->pfcorr.as<float>(),
-                        nullptr, nullptr, nullptr, c->st);
-    launch_w4a8_gemm(m.a8w.as<uint4>(), m.a8s.as<uint4>(), c->pfxq.as<uint16_t>(), c->pfsx.as<float>(),
-                     c->pfcorr.as<float>(), y, M, m.N, m.K, m.N, c->st);
+    const A8Rows q = pf_rows(c, M, set);
+    if (quant || M <= 8) launch_w4a8_quant(x, M, q.ld, m.K, q.q, q.sx, q.corr, nullptr, nullptr, nullptr, c->st);
+    launch_w4a8_gemm(m.a8w.as<uint4>(), m.a8s.as<uint4>(), q.q, q.sx, q.corr, y, M, m.N, m.K, m.N, c->st);
   } else {  // exact float: the matrix-core GEMM past MAXM rows, else the GEMV
     const Mat* mp = &m;
     if (!pf_exact(c, 1, &mp, x, M, &y, false)) launch_gemv(plain_args(m, x, y, M), EPI_STORE, c->st);
@@ -1798,13 +1804,15 @@ static void pf_lin(g4v_ctx* c, const Mat& m, const float* x, int M, float* y, bo
 }
 
 // up to three products of the same input (same K) in one launch: q / k / v, gate / up
-static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x, int M, float* const* y, bool i8) {
+// (quant = false: x's quantised rows are there, as for pf_lin; pair, i8 and M > 8: gate and up, the
+// activation to the second set of quantised rows)
+static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x, int M, float* const* y, bool i8,
+                         bool quant = true, bool pair = false) {
   if (i8) {
-    bool n16 = true;
-    for (int j = 0; j < n; ++j) n16 = n16 && m[j]->N % 16 == 0;
-    if (M <= 8 && n16) {  // decode rows: the n products in one launch (i8_task over nj matrices, E:303-309)
+    if (quant || M <= 8)
       launch_w4a8_quant(x, M, w4a8_mpad(M), m[0]->K, c->pfxq.as<uint16_t>(), c->pfsx.as<float>(),
                         c->pfcorr.as<float>(), nullptr, nullptr, nullptr, c->st);
+    if (M <= 8) {  // decode rows: the n products in one launch (i8_task over nj matrices, E:303-309)
       A8Dec d{};
       for (int j = 0; j < n; ++j) {
         d.tw[j] = m[j]->a8w.as<uint4>();
@@ -1814,11 +1822,20 @@ static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x,
         d.t0[j + 1] = d.t0[j] + m[j]->N / 16;
       }
       for (int j = n + 1; j < 4; ++j) d.t0[j] = d.t0[n];
-      if (launch_w4a8_dec(d, n, c->pfxq.as<uint16_t>(), c->pfsx.as<float>(), c->pfcorr.as<float>(), M, m[0]->K,
-                          c->st))
-        return;
+      (void)launch_w4a8_dec(d, n, c->pfxq.as<uint16_t>(), c->pfsx.as<float>(), c->pfcorr.as<float>(), M, m[0]->K,
+                            c->st);
+      return;
     }
-    for (int j = 0; j < n; ++j) pf_lin(c, *m[j], x, M, y[j], true, j == 0);
+    A8Gemm q{};
+    for (int j = 0; j < n; ++j) {
+      q.tw[j] = m[j]->a8w.as<uint4>();
+      q.ts[j] = m[j]->a8s.as<uint4>();
+      q.y[j] = y[j];
+      q.ldy[j] = q.N[j] = m[j]->N;
+    }
+    if (pair) q.yq = pf_rows(c, M, 1);
+    (void)launch_w4a8_gemm_multi(q, n, pair, c->pfxq.as<uint16_t>(), c->pfsx.as<float>(), c->pfcorr.as<float>(), M,
+                                 m[0]->K, c->st);
     return;
   }
   if (pf_exact(c, n, m, x, M, y, false)) return;
@@ -1834,15 +1851,21 @@ static void pf_lin_multi(g4v_ctx* c, int n, const Mat* const* m, const float* x,
   launch_gemv(a, EPI_STORE, c->st);
 }
 
-// gate, up and the activation act = r16(r16(gelu8(r16 g)) * r16 u) (E:1363-1371)
-static void pf_gate_up(g4v_ctx* c, const Mat& mg, const Mat& mu, const float* x, int M, float* gb, float* ub,
-                       float* act, bool i8) {
+// gate, up, the activation act = r16(r16(gelu8(r16 g)) * r16 u) and down (E:1363-1373).  x: the rows,
+// or with W4A8 and more than 8 of them their quantised form in pf_rows
+static void pf_mlp(g4v_ctx* c, const Mat& mg, const Mat& mu, const Mat& md, const float* x, int M, float* gb,
+                   float* ub, float* act, float* o, bool i8) {
   const Mat* m[2] = {&mg, &mu};
   float* ya[2] = {act, act};
-  if (!i8 && pf_exact(c, 2, m, x, M, ya, true)) return;
-  float* yg[2] = {gb, ub};
-  pf_lin_multi(c, 2, m, x, M, yg, i8);
-  launch_pf_act(gb, ub, act, (size_t)M * mg.N, c->st);
+  const bool many = i8 && M > 8;
+  if (many) {
+    pf_lin_multi(c, 2, m, x, M, ya, true, false, true);
+  } else if (i8 || !pf_exact(c, 2, m, x, M, ya, true)) {
+    float* yg[2] = {gb, ub};
+    pf_lin_multi(c, 2, m, x, M, yg, i8);
+    launch_pf_act(gb, ub, act, (size_t)M * mg.N, c->st);
+  }
+  pf_lin(c, md, act, M, o, i8, !many, many ? 1 : 0);
 }
 
 static int pf_alloc(g4v_ctx* c, int rows, size_t sfl) {
@@ -1861,6 +1884,9 @@ static int pf_alloc(g4v_ctx* c, int rows, size_t sfl) {
     ALLOC(c->pfxq, Rp * Kmax * 2);
     ALLOC(c->pfsx, (Kmax / 32) * Rp * 4);
     ALLOC(c->pfcorr, (Kmax / 32) * Rp * 4);
+    ALLOC(c->pfxq2, Rp * c->I * 2);
+    ALLOC(c->pfsx2, (c->I / 32) * Rp * 4);
+    ALLOC(c->pfcorr2, (c->I / 32) * Rp * 4);
     ALLOC(c->pftok, R * 4);
     if (!c->pfh.p) ALLOC(c->pfh, H * 4);
     c->pf_rows = rows;
@@ -1886,7 +1912,8 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
   float *gb = c->pfg.as<float>() + off * c->I, *ub = c->pfu.as<float>() + off * c->I,
         *act = c->pfact.as<float>() + off * c->I;
   const int P0 = g.pos0 + r0;
-  launch_pf_embed(c->E.as<uint16_t>(), c->pftok.as<int>() + r0, c->L[0]->ln().in_ln, sqh, x, a, M, st);
+  const A8Rows aq = pf_out(c, M, i8);  // the products' inputs leave the kernels before them quantised
+  launch_pf_embed(c->E.as<uint16_t>(), c->pftok.as<int>() + r0, c->L[0]->ln().in_ln, sqh, x, a, M, st, aq);
   for (int l = 0; l < c->NL; ++l) {
     const Layer& lay = *c->L[l];
     const LayerNorms ln = lay.ln();
@@ -1896,7 +1923,7 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
     {  // E:1289
       const Mat* mq[3] = {&lay.m[0], &lay.m[1], &lay.m[2]};
       float* yq[3] = {q, k, v};
-      pf_lin_multi(c, 3, mq, a, M, yq, i8);
+      pf_lin_multi(c, 3, mq, a, M, yq, i8, false);
     }
     const float* cs = c->rope.as<float>() + (size_t)(2 * ty) * c->ctxcap * (HD / 2);
     const float* sn = cs + (size_t)c->ctxcap * (HD / 2);
@@ -1918,15 +1945,14 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
                        NQ * HD, st);
     } else {
       launch_pf_attn(c->pfq.as<float>(), KCl, VCl, c->pfs.as<float>(), c->pfatt.as<float>(), g, r0, M, lay.sliding,
-                     st);
+                     st, false, HD, nullptr, 0, aq);
     }
-    pf_lin(c, lay.m[3], att, M, o, i8, true);  // E:1356
-    launch_pf_post_attn(o, x, a, ln.post_attn, ln.pre_ff, M, st);
-    pf_gate_up(c, lay.m[4], lay.m[5], a, M, gb, ub, act, i8);  // E:1366-1371
-    pf_lin(c, lay.m[6], act, M, o, i8, true);  // E:1373
+    pf_lin(c, lay.m[3], att, M, o, i8, false);  // E:1356
+    launch_pf_post_attn(o, x, a, ln.post_attn, ln.pre_ff, M, st, aq);
+    pf_mlp(c, lay.m[4], lay.m[5], lay.m[6], a, M, gb, ub, act, o, i8);  // E:1366-1373
     const bool lastl = l + 1 == c->NL;
     launch_pf_post_ff(o, x, a, ln.post_ff, lastl ? nullptr : c->L[l + 1]->ln().in_ln, c->fnorm.as<float>(),
-                      lay.scalar, c->pfh.as<float>(), lastl ? hrow : -1, M, st);
+                      lay.scalar, c->pfh.as<float>(), lastl ? hrow : -1, M, st, nullptr, lastl ? A8Rows{} : aq);
   }
 }
 
@@ -1986,6 +2012,9 @@ int gm_reserve(g4v_ctx* c, int rows, size_t sfl) {
     ALLOC(c->pfxq, Rp * Kmax * 2);
     ALLOC(c->pfsx, (Kmax / 32) * Rp * 4);
     ALLOC(c->pfcorr, (Kmax / 32) * Rp * 4);
+    ALLOC(c->pfxq2, Rp * c->gm_Imax * 2);
+    ALLOC(c->pfsx2, (c->gm_Imax / 32) * Rp * 4);
+    ALLOC(c->pfcorr2, (c->gm_Imax / 32) * Rp * 4);
     c->gm_cap = rows;
   }
   if (sfl > c->gm_sfl) {
@@ -2050,6 +2079,7 @@ void gm_forward(g4v_ctx* c, int M, int pos0, int nsplit, int sib, int hrow, bool
   AttnGeom* geo = c->gm_geo.as<AttnGeom>();
   if (spd && split) launch_step_geom(spd, nsplit, geo, st);
   i8 = i8 && M >= 2;  // lin_multi's rule (E:311)
+  const A8Rows aq = pf_out(c, M, i8);  // the products' inputs leave the kernels before them quantised
   launch_pf_embed(c->E.as<uint16_t>(), tok, c->gm[0].nv.as<float>(), sqh, R.x, R.a, M, st);  // E:1262-1267
   pf_lin(c, c->gm_plproj, R.x, M, R.pr, i8, true);                                            // E:615-660
   launch_gm_ple(R.pr, tok, c->gm_ple.as<uint16_t>(), c->gm_plnorm.as<float>(), R.pli, M, st);
@@ -2067,7 +2097,7 @@ void gm_forward(g4v_ctx* c, int M, int pos0, int nsplit, int sib, int hrow, bool
     {  // E:1287-1288: q (and k, v on the owner layers) in one launch
       const Mat* mq[3] = {&lay.m[0], &lay.m[1], &lay.m[2]};
       float* yq[3] = {R.q, R.k, R.v};
-      pf_lin_multi(c, own ? 3 : 1, mq, R.a, M, yq, i8);
+      pf_lin_multi(c, own ? 3 : 1, mq, R.a, M, yq, i8, l == 0);
     }
     const float* cs = ty ? c->gm_rope.as<float>() : c->rope.as<float>();
     const float* sn = cs + (size_t)c->ctxcap * (hd / 2);
@@ -2102,20 +2132,19 @@ void gm_forward(g4v_ctx* c, int M, int pos0, int nsplit, int sib, int hrow, bool
                          NQ * HD, st);
     } else {  // attn_tile (M >= 4 past 64 keys, no sibling) or run_mh: one block of M rows
       launch_pf_attn(R.q, KCo, VCo, c->gm_s.as<float>(), R.att, pg ? *pg : PfGeom{M, pos0, M, sib}, 0, M, sliding,
-                     st, false, hd, dpos, c->ctxcap);
+                     st, false, hd, dpos, c->ctxcap, aq);
     }
     if (split) pmark(c, PT_ATTN, 0, 0);
-    pf_lin(c, lay.m[3], R.att, M, R.o, i8, true);                       // E:1356
-    launch_pf_post_attn(R.o, R.x, R.a, post_attn, pre_ff, M, st);       // E:1358-1361
-    pf_gate_up(c, lay.m[4], lay.m[5], R.a, M, R.g, R.u, R.act, i8);  // E:1363-1371
-    pf_lin(c, lay.m[6], R.act, M, R.o, i8, true);                                               // E:1373
-    launch_pf_post_ff(R.o, R.x, R.a, post_ff, nullptr, nullptr, 1.0f, nullptr, -1, M, st);      // E:1375-1377
-    pf_lin(c, G.pg, R.x, M, R.pgv, i8, true);                                                   // E:1379-1384
+    pf_lin(c, lay.m[3], R.att, M, R.o, i8, false);                          // E:1356
+    launch_pf_post_attn(R.o, R.x, R.a, post_attn, pre_ff, M, st, aq);       // E:1358-1361
+    pf_mlp(c, lay.m[4], lay.m[5], lay.m[6], R.a, M, R.g, R.u, R.act, R.o, i8);  // E:1363-1373
+    launch_pf_post_ff(R.o, R.x, R.a, post_ff, nullptr, nullptr, 1.0f, nullptr, -1, M, st, nullptr, aq);      // E:1375-1377
+    pf_lin(c, G.pg, R.x, M, R.pgv, i8, false);                                                   // E:1379-1384
     launch_gm_pg_act(R.pgv, R.pli, l, M, R.g2, st);
     pf_lin(c, G.pp, R.g2, M, R.o, i8, true);                                                    // E:1386
     const bool last = l + 1 == GM_NL;                                                           // E:1387-1404
     launch_pf_post_ff(R.o, R.x, R.a, post_ple, last ? nullptr : c->gm[l + 1].nv.as<float>(), c->fnorm.as<float>(),
-                      G.scalar, h, last ? hrow : -1, M, st, hn);
+                      G.scalar, h, last ? hrow : -1, M, st, hn, last ? A8Rows{} : aq);
   }
 }
 
@@ -2414,7 +2443,7 @@ int g4v_model_create_gemma(g4v_ctx* c, int V, const int* mlp, int ctxcap) {
   }
   c->gm_cap = 0;
   c->gm_sfl = 0;
-  r = gm_reserve(c, GM_ROWS, (size_t)pf_score_floats(GM_ROWS, ctxcap, 0));  // a prompt block / verify pass
+  r = gm_reserve(c, GM_ROWS, (size_t)pf_score_floats(GM_ROWS, ctxcap));  // a prompt block / verify pass
   if (r) return r;
   ALLOC(c->po5, (size_t)MAXT * MAXM * NQ * 512 * 4);
   ALLOC(c->pm5, (size_t)MAXT * MAXM * NQ * 4);
@@ -2691,7 +2720,7 @@ static int gm_prefill(g4v_ctx* c, const int* toks, int n, int pos0, int pfb, int
          "prefill: more positions per split than the split buffer holds");
   HIPCHK(hipSetDevice(c->device));
   if (nA > 0) {
-    int r = gm_reserve(c, nA, (size_t)pf_score_floats(nA, pos0, 0));
+    int r = gm_reserve(c, nA, (size_t)pf_score_floats(nA, pos0));
     if (r) return r;
     HIPCHK(hipMemcpyAsync(c->gm_tok.p, toks, (size_t)nA * 4, hipMemcpyHostToDevice, c->st));
     const PfGeom g{n, pos0, pfb, -1};
@@ -2747,11 +2776,8 @@ extern "C" int g4v_prefill(g4v_ctx* c, const int* toks, int n, int pos0, int pfb
   const int nA = tail ? n - Ml : n;
   if (tsplit)
     ARGCHK((Ml + p0l + nsplit - 1) / nsplit <= attn_pmax(), "prefill: more positions per split than the split buffer holds");
-  size_t sfl = 0;
-  for (int l = 0; l < c->NL; ++l) {
-    sfl = std::max(sfl, (size_t)pf_score_floats(nA, pos0, c->L[l]->sliding));
-    if (tail && !tsplit) sfl = std::max(sfl, (size_t)pf_score_floats(Ml, p0l, c->L[l]->sliding));
-  }
+  size_t sfl = (size_t)pf_score_floats(nA, pos0);
+  if (tail && !tsplit) sfl = std::max(sfl, (size_t)pf_score_floats(Ml, p0l));
   int r = pf_alloc(c, n, sfl);
   if (r) return r;
   HIPCHK(hipMemcpyAsync(c->pftok.p, toks, (size_t)n * 4, hipMemcpyHostToDevice, c->st));
@@ -2818,6 +2844,22 @@ constexpr size_t DR_SCRATCH_BYTES = (size_t)(5 * DR_H + 2 * DR_Q * DR_HDMAX + DR
                                     (size_t)(32 + 16 + 16 + DR_IN_WORDS) * 4 + 16 * sizeof(AttnGeom);
 }  // namespace
 
+// the drafter's matrices, as generated or loaded, into the layout its products read
+static void dr_chains(g4v_ctx* c) {
+  hipStream_t st = c->st;
+  launch_b16_chains(c->dr_pre.as<uint16_t>(), DR_H, 2 * H, st);
+  launch_b16_chains(c->dr_post.as<uint16_t>(), H, DR_H, st);
+  launch_b16_chains(c->dr_cent.as<uint16_t>(), c->V / 128, DR_H, st);
+  launch_b16_chains(c->dr_emb.as<uint16_t>(), c->V, DR_H, st);
+  for (int l = 0; l < 4; ++l) {
+    launch_b16_chains(c->dr_q[l].as<uint16_t>(), DR_Q * c->dr_hd[l], DR_H, st);
+    launch_b16_chains(c->dr_o[l].as<uint16_t>(), DR_H, DR_Q * c->dr_hd[l], st);
+    launch_b16_chains(c->dr_g[l].as<uint16_t>(), DR_F, DR_H, st);
+    launch_b16_chains(c->dr_u[l].as<uint16_t>(), DR_F, DR_H, st);
+    launch_b16_chains(c->dr_d[l].as<uint16_t>(), DR_H, DR_F, st);
+  }
+}
+
 extern "C" int g4v_drafter_synth(g4v_ctx* c, uint64_t seed) {
   if (!c) return G4V_E_ARG;
   if (!c->model_ready) {
@@ -2844,22 +2886,6 @@ extern "C" int g4v_drafter_synth(g4v_ctx* c, uint64_t seed) {
     launch_gen_bf16_normal(b.as<uint16_t>(), n, rng_stream(seed, tag), scale, st);
     return 0;
   };
-// the drafter's matrices, as generated or loaded, into the layout its products read
-static void dr_chains(g4v_ctx* c) {
-  hipStream_t st = c->st;
-  launch_b16_chains(c->dr_pre.as<uint16_t>(), DR_H, 2 * H, st);
-  launch_b16_chains(c->dr_post.as<uint16_t>(), H, DR_H, st);
-  launch_b16_chains(c->dr_cent.as<uint16_t>(), c->V / 128, DR_H, st);
-  launch_b16_chains(c->dr_emb.as<uint16_t>(), c->V, DR_H, st);
-  for (int l = 0; l < 4; ++l) {
-    launch_b16_chains(c->dr_q[l].as<uint16_t>(), DR_Q * c->dr_hd[l], DR_H, st);
-    launch_b16_chains(c->dr_o[l].as<uint16_t>(), DR_H, DR_Q * c->dr_hd[l], st);
-    launch_b16_chains(c->dr_g[l].as<uint16_t>(), DR_F, DR_H, st);
-    launch_b16_chains(c->dr_u[l].as<uint16_t>(), DR_F, DR_H, st);
-    launch_b16_chains(c->dr_d[l].as<uint16_t>(), DR_H, DR_F, st);
-  }
-}
-
   int r;
   if ((r = gen(c->dr_pre, (size_t)DR_H * 2 * H, 5000, 0.02f))) return r;
   for (int l = 0; l < 4; ++l) {
@@ -2894,6 +2920,7 @@ static void dr_chains(g4v_ctx* c) {
   ALLOC(c->dr_s, DR_SCRATCH_BYTES);
   HIPCHK(hipMemcpyAsync(c->dr_norms.p, nv.data(), nv.size() * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(c->dr_order.p, order.data(), (size_t)V * 4, hipMemcpyHostToDevice, st));
+  dr_chains(c);
   HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));
   c->dr_C = C;
@@ -2920,7 +2947,6 @@ extern "C" int g4v_drafter_load(g4v_ctx* c, const g4v_drafter_tensors* t) {
   for (int l = 0; l < 4; ++l) {
     ARGCHK(t->q[l] && t->o[l] && t->gate[l] && t->up[l] && t->down[l], "drafter_load: null tensor");
     for (int k = 0; k < 5; ++k) ARGCHK(t->nv[l][k], "drafter_load: null norm");
-  dr_chains(c);
   }
   for (long long i = 0; i < V; ++i)
     ARGCHK(t->order[i] >= 0 && t->order[i] < V, "drafter_load: token ordering outside the vocabulary");
@@ -2964,6 +2990,8 @@ extern "C" int g4v_drafter_load(g4v_ctx* c, const g4v_drafter_tensors* t) {
   ALLOC(c->dr_s, DR_SCRATCH_BYTES);
   HIPCHK(hipMemcpyAsync(c->dr_norms.p, nv.data(), nv.size() * 4, hipMemcpyHostToDevice, st));
   HIPCHK(hipMemcpyAsync(c->dr_order.p, order.data(), (size_t)V * 4, hipMemcpyHostToDevice, st));
+  dr_chains(c);
+  HIPCHK(hipGetLastError());
   HIPCHK(hipStreamSynchronize(st));
   c->dr_C = C;
   c->dr_ready = true;
@@ -2990,8 +3018,6 @@ static void enqueue_draft(g4v_ctx* c, int k, int nsplit) {
       L.E = c->E.as<uint16_t>(), L.tok = d.tok + j;
       launch_b16(L, st);
     }
-  dr_chains(c);
-  HIPCHK(hipGetLastError());
     for (int l = 0; l < 4; ++l) {
       const bool sliding = l < 3;
       const int ty = sliding ? 0 : 1, ol = sliding ? 13 : 14, hd = c->dr_hd[l];  // E:1540

@@ -485,6 +485,19 @@ struct A8Dec {
 };
 int launch_w4a8_dec(const A8Dec& m, int n, const uint16_t* xqb, const float* sxt, const float* corr, int M, int K,
                     hipStream_t st);
+// products of more than 8 quantised rows over up to three matrices of one input (N_j % 16 == 0,
+// K % 256 == 0); pair: matrices 0 and 1 are gate and up and y[0] receives the activation.  0: refused.
+struct A8Gemm {
+  const uint4* tw[3];
+  const uint4* ts[3];
+  float* y[3];
+  int ldy[3];
+  int N[3];
+  int t0[4];  // set by the launch
+  A8Rows yq;  // pair: the activation's quantised rows instead of y[0] (yq.q not null, N % 32 == 0)
+};
+int launch_w4a8_gemm_multi(const A8Gemm& q, int n, bool pair, const uint16_t* xqb, const float* sxt, const float* corr,
+                           int M, int K, hipStream_t st);
 void launch_w4a8_gemm(const uint4* tw, const uint4* ts, const uint16_t* xqb, const float* sxt, const float* corr,
                       float* y, int M, int N, int K, int ldy, hipStream_t st);
 // exact-order products of many rows (g4v_gemmx.hip) on the W4A8 operand tiles: up to three matrices

@@ -140,28 +140,34 @@ void launch_gen_w4(uint8_t* w, uint16_t* s, size_t nbytes, size_t nscales, uint6
 struct PfGeom {
   int n, pos0, pfb, sib;
 };
+// (aq.q not null: the next product's input, a, leaves quantised instead of as floats)
 void launch_pf_embed(const uint16_t* E, const int* toks, const float* in_ln, float sqh, float* x, float* a, int M,
-                     hipStream_t st);
+                     hipStream_t st, const A8Rows& aq = A8Rows{});
 // q [M][8 hd] normed + rotated in place; k, v [M][hd] normed into the cache rows P0 .. (own = 0:
 // q only, the layer reads another layer's cache); row sib (>= 0) is rotated at position P0 + 1
 // (the sibling row).  hd 256 or 512; cs / sn the layer type's RoPE tables [ctx][hd / 2].
 void launch_pf_qkv(float* q, const float* k, const float* v, const float* qn, const float* kn, const float* cs,
                    const float* sn, uint16_t* KC, uint16_t* VC, int P0, int M, hipStream_t st, int sib = -1,
                    int hd = HD, int own = 1, const int* dpos = nullptr);
-// score scratch (floats) of M rows starting at position Pb
-long long pf_score_floats(int M, int Pb, int sliding);
+// score scratch (floats) of up to M rows starting at position Pb, on either layer type
+long long pf_score_floats(int M, int Pb);
+// attention of more than MAXM prompt rows (g4v_pfattn.hip), and its scratch
+void launch_pfa(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g, int r0,
+                int M, int sliding, hipStream_t st, int hd, const A8Rows& aq);
+long long pfa_scratch_floats(int M, int Pb);
 // attn_tile / run_mh attention of segment rows [r0, r0 + M): q [n][2048] (row r at r), att likewise
 // staged: att rows in the staged GEMV input layout (staged_index) instead of plain.
 // dpos (launch_pf_qkv too): not null, g.pos0 (P0) is read from that device word when the kernels
 // run, so that a captured pass serves every position; the grid then covers positions below maxpos.
 void launch_pf_attn(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g,
                     int r0, int M, int sliding, hipStream_t st, bool staged = false, int hd = HD,
-                    const int* dpos = nullptr, int maxpos = 0);
-void launch_pf_post_attn(const float* o, float* x, float* a, const float* w1, const float* w2, int M, hipStream_t st);
+                    const int* dpos = nullptr, int maxpos = 0, const A8Rows& aq = A8Rows{});
+void launch_pf_post_attn(const float* o, float* x, float* a, const float* w1, const float* w2, int M, hipStream_t st,
+                         const A8Rows& aq = A8Rows{});
 void launch_pf_act(const float* g, const float* u, float* act, size_t n, hipStream_t st);
 void launch_pf_post_ff(const float* o, float* x, float* a, const float* w1, const float* next_in_ln,
                        const float* fnorm, float scalar, float* h, int hrow, int M, hipStream_t st,
-                       float* hn = nullptr);
+                       float* hn = nullptr, const A8Rows& aq = A8Rows{});
 // the per-layer-input branch of the Gemma-4-E2B layout: pli [M][35][256] from the projection rows
 // pr [M][35 * 256] (E:615-660); g2 [M][256] for layer l from the gate rows pgv (E:405-443)
 void launch_gm_ple(const float* pr, const int* toks, const uint16_t* ple, const float* plnorm, float* pli, int M,
@@ -197,14 +203,14 @@ struct B16Launch {
   int pro = 0, epi = 0;
 };
 void launch_b16(const B16Launch& L, hipStream_t st);
+// a bf16 matrix [rows][K] into the chain-major rows launch_b16 reads, in place (K % 128 == 0, K <= 3072)
+void launch_b16_chains(uint16_t* W, int rows, int K, hipStream_t st);
 // q heads normed and rotated at position *Pp + 1 + j
 void launch_dr_qnorm(float* q, const float* qn, const float* cs, const float* sn, const int* Pp, int j, int hd,
                      hipStream_t st);
 // a chain's inputs: in = {tok, P, hrow, _, h[1536]}; hin = h (hrow < 0) or hbase row hrow;
 // tok[0] = tok; geo[2 j + s] = the attention geometry of step j on sliding (s = 0) / global layers
 void launch_dr_setup(const int* in, const float* hbase, float* hin, int* tok, AttnGeom* geo, int k, int T,
-// a bf16 matrix [rows][K] into the chain-major rows launch_b16 reads, in place (K % 128 == 0, K <= 3072)
-void launch_b16_chains(uint16_t* W, int rows, int K, hipStream_t st);
                      hipStream_t st);
 void launch_dr_rank(const float* score, int C, int* top, hipStream_t st);
 void launch_dr_best(const float* cs, const int* top, const int* order, int nc, int* tok, int* sec, float* gap,

@@ -9,12 +9,12 @@
 // The linear layers are the W4A8 matrix-core GEMM (g4v_w4a8.hip); the row kernels below hold the
 // norms, RoPE, cache writes and residuals in plain [row][K] layouts.
 //
-// Prefill attention, per row r at position P (lo = P - 511 clamped at 0 on sliding layers, else
+// Attention of up to MAXM rows (prompts: g4v_pfattn.hip), per row r at position P (lo = P - 511 clamped at 0 on sliding layers, else
 // 0) and query head h, with K, V in the device cache layout (kc_index / vc_index):
 //   scores (k_pf_scores): s_p = q . k_p in the path's chain order (attn_tile: two 8-lane FMA
 //     chains over hd in steps of 16, summed lane-wise, then hsum; run_mh: one 8-lane chain in
 //     steps of 8, then hsum), written to a scratch row [8][P - lo + 1];
-//   output (k_pf_attn_out): mx = max_p s_p; attn_tile: w = exp8(s - mx), den = sum w in order,
+//   output (k_pf_attn_rows): mx = max_p s_p; attn_tile: w = exp8(s - mx), den = sum w in order,
 //     O = fma(w, v, O) in position order, out = r16(O * (1 / den)); run_mh: e = expf(s - mx),
 //     den = sum e in order, O = fma(e / den, v, O) in order, out = r16(O).
 #include <algorithm>
@@ -53,10 +53,12 @@ __device__ __forceinline__ long long pf_srow(int rr, int r, int nrows, int Pb, i
   return r == g.sib ? pf_soff(nrows, Pb, sliding) : pf_soff(rr, Pb, sliding);
 }
 
+// The row kernels below that form a product's input a write it as floats or, with aq.q set (a W4A8
+// product of many rows), quantised (a8_store_row), which saves its trip through memory and a launch.
 // E:1262-1267: x = r16(E[tok] * sqrt(H)); a = (x * r) * in_ln (unrounded: the W4A8 source)
 __global__ __launch_bounds__(ROW_THREADS) void k_pf_embed(const uint16_t* __restrict__ E, const int* __restrict__ toks,
                                                           const float* __restrict__ in_ln, float sqh,
-                                                          float* __restrict__ x, float* __restrict__ a) {
+                                                          float* __restrict__ x, float* __restrict__ a, A8Rows aq) {
   __shared__ __align__(16) float xs[H];
   __shared__ double red[16];
   const int m = blockIdx.x;
@@ -245,168 +247,9 @@ __global__ __launch_bounds__(256) void k_pf_scores(const float* __restrict__ q, 
   for (int h = 0; h < NQ; ++h) Srow[(size_t)h * len + (p - lo)] = ok ? hsum8(vv[h]) : -INFINITY;
 }
 
-// output of one row: one wave, lane l holds dims 4l .. 4l+3 of the 8 heads (32 accumulators), so
-// each weight read from LDS (wave-uniform) feeds 4 FMAs.  Weights of PF_CP positions at a time
-// go to LDS; the value rows are read 8 positions (16 bytes of a dim) at a time where positions
-// are 8-aligned, one at a time at the edges of the range
-constexpr int PF_CP = 256;  // positions per weight chunk (4 per lane)
-template <int D>
-__global__ __launch_bounds__(64) void k_pf_attn_out(const float* __restrict__ S, const uint16_t* __restrict__ VC,
-                                                    float* __restrict__ att, PfGeom g, int r0, int sliding,
-                                                    ExpfTab tab, int staged, const int* __restrict__ dpos) {
-  __shared__ __align__(16) float w[NQ][PF_CP];
-  if (dpos) g.pos0 = *dpos;
-  __shared__ uint64_t T[32];
-  // the last rows (longest ranges) first, so that the long blocks do not trail the grid
-  const int rr = gridDim.x - 1 - blockIdx.x, r = r0 + rr, P = g.pos0 + r, lo = pf_row_lo(r, P, g, sliding);
-  const int len = P - lo + 1;
-  const int lane = threadIdx.x;
-  const bool tiled = pf_tiled(r, g);
-  const float* Srow = S + pf_srow(rr, r, gridDim.x, g.pos0 + r0, sliding, g);
-  if (lane < 32) T[lane] = tab.t[lane];
-  float mx[NQ];  // max per head (order-free), on every lane
-#pragma unroll
-  for (int h = 0; h < NQ; ++h) {
-    float m = -1e30f;
-    for (int jj = lane; jj < len; jj += 64) m = fmaxf(m, Srow[(size_t)h * len + jj]);
-#pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) m = fmaxf(m, __shfl_xor(m, o));
-    mx[h] = m;
-  }
-  __syncthreads();  // T
-  float den = 0.f;  // lanes 0..7: head `lane`'s sum in position order
-  if (!tiled) {     // run_mh divides by the sum before the V pass
-    for (int c0 = 0; c0 < len; c0 += PF_CP) {
-      const int cn = min(PF_CP, len - c0);
-#pragma unroll
-      for (int k = 0; k < PF_CP / 64; ++k) {
-        const int jj = lane + 64 * k;
-        if (jj < cn) {
-          const bool ok = pf_valid(r, P, lo + c0 + jj, g);  // skipped positions weigh 0 (den + 0 is exact)
-#pragma unroll
-          for (int h = 0; h < NQ; ++h) w[h][jj] = ok ? libm_expf_neg(Srow[(size_t)h * len + c0 + jj] - mx[h], T) : 0.f;
-        }
-      }
-      __syncthreads();
-      if (lane < NQ)
-        for (int jj = 0; jj < cn; ++jj) den = den + w[lane][jj];
-      __syncthreads();
-    }
-  }
-  float dh[NQ];  // run_mh: the sums, on every lane
-#pragma unroll
-  for (int h = 0; h < NQ; ++h) dh[h] = __shfl(den, h);
-  constexpr int DL = D / 64;  // dims per lane
-  float O[NQ][DL];
-#pragma unroll
-  for (int h = 0; h < NQ; ++h)
-#pragma unroll
-    for (int d = 0; d < DL; ++d) O[h][d] = 0.f;
-  // dim DL lane + d of position p in the cache layout (vc_index_d)
-  auto vat = [&](int p, int d) { return VC + vc_index_d<D>(p, DL * lane + d); };
-  float sreg[PF_CP / 64][NQ];  // scores of this lane's positions of the next chunk
-#pragma unroll
-  for (int k = 0; k < PF_CP / 64; ++k)
-#pragma unroll
-    for (int h = 0; h < NQ; ++h) sreg[k][h] = lane + 64 * k < len ? Srow[(size_t)h * len + lane + 64 * k] : 0.f;
-  for (int c0 = 0; c0 < len; c0 += PF_CP) {
-    const int cn = min(PF_CP, len - c0);
-#pragma unroll
-    for (int k = 0; k < PF_CP / 64; ++k) {
-      const int jj = lane + 64 * k;
-      if (jj < cn) {
-        const bool ok = pf_valid(r, P, lo + c0 + jj, g);  // fma(0, v, O) leaves O as it is
-#pragma unroll
-        for (int h = 0; h < NQ; ++h) {
-          const float dd = sreg[k][h] - mx[h];
-          w[h][jj] = !ok ? 0.f : (tiled ? exp8(dd) : libm_expf_neg(dd, T) / dh[h]);
-        }
-      }
-    }
-    __syncthreads();
-#pragma unroll
-    for (int k = 0; k < PF_CP / 64; ++k) {
-      const int jj = c0 + PF_CP + lane + 64 * k;
-      if (jj < len)
-#pragma unroll
-        for (int h = 0; h < NQ; ++h) sreg[k][h] = Srow[(size_t)h * len + jj];
-    }
-    const int pa = lo + c0, pe = pa + cn;  // positions [pa, pe) of this chunk
-    const int a8 = min((pa + 7) & ~7, pe), e8 = max(pe & ~7, a8);
-    for (int p = pa; p < a8; ++p) {        // leading positions up to an 8-boundary
-      float v[DL];
-#pragma unroll
-      for (int d = 0; d < DL; ++d) v[d] = bf2f(*vat(p, d));
-#pragma unroll
-      for (int h = 0; h < NQ; ++h) {
-        const float ww = w[h][p - pa];
-#pragma unroll
-        for (int d = 0; d < DL; ++d) O[h][d] = fmaf(ww, v[d], O[h][d]);
-      }
-    }
-    for (int p = a8; p < e8; p += 8) {     // 8 positions of each of the lane's 4 dims
-      uint4 vq[DL];
-#pragma unroll
-      for (int d = 0; d < DL; ++d) vq[d] = *reinterpret_cast<const uint4*>(vat(p, d));
-      const int j0 = p - pa;
-#pragma unroll
-      for (int t2 = 0; t2 < 4; ++t2) {     // positions j0 + 2 t2, j0 + 2 t2 + 1
-        float va[DL], vb[DL];
-#pragma unroll
-        for (int d = 0; d < DL; ++d) {
-          const uint32_t u = t2 == 0 ? vq[d].x : (t2 == 1 ? vq[d].y : (t2 == 2 ? vq[d].z : vq[d].w));
-          va[d] = as_f32(u << 16);
-          vb[d] = as_f32(u & 0xFFFF0000u);
-        }
-#pragma unroll
-        for (int h = 0; h < NQ; ++h) {
-          const float wa = w[h][j0 + 2 * t2], wb = w[h][j0 + 2 * t2 + 1];  // j0 may be odd
-#pragma unroll
-          for (int d = 0; d < DL; ++d) O[h][d] = fmaf(wa, va[d], O[h][d]);
-#pragma unroll
-          for (int d = 0; d < DL; ++d) O[h][d] = fmaf(wb, vb[d], O[h][d]);
-        }
-      }
-    }
-    for (int p = e8; p < pe; ++p) {        // trailing positions
-      float v[DL];
-#pragma unroll
-      for (int d = 0; d < DL; ++d) v[d] = bf2f(*vat(p, d));
-#pragma unroll
-      for (int h = 0; h < NQ; ++h) {
-        const float ww = w[h][p - pa];
-#pragma unroll
-        for (int d = 0; d < DL; ++d) O[h][d] = fmaf(ww, v[d], O[h][d]);
-      }
-    }
-    if (tiled && lane < NQ)
-      for (int jj = 0; jj < cn; ++jj) den = den + w[lane][jj];
-    __syncthreads();
-  }
-  const float inv = tiled ? 1.0f / den : 1.0f;  // lanes 0..7
-  float* orow = att + (size_t)r * NQ * D;
-#pragma unroll
-  for (int h = 0; h < NQ; ++h) {
-    const float ih = __shfl(inv, h);
-    float v[DL];
-#pragma unroll
-    for (int d = 0; d < DL; ++d) v[d] = tiled ? r16(O[h][d] * ih) : r16(O[h][d]);
-    const int n0 = h * D + DL * lane;
-    if (staged) {  // the staged GEMV input layout of the o projection (staged_index)
-#pragma unroll
-      for (int d = 0; d < DL; ++d) orow[staged_index(n0 + d)] = v[d];
-    } else {
-#pragma unroll
-      for (int d4 = 0; d4 < DL; d4 += 4)
-        *reinterpret_cast<float4*>(orow + n0 + d4) = make_float4(v[d4], v[d4 + 1], v[d4 + 2], v[d4 + 3]);
-    }
-  }
-}
-
-// The same output for a pass of few rows (a verify pass, M <= 8): one block per (row, head), one
-// output dim per thread, so that every dim's chain over the positions has a thread of its own
-// (the kernel above gives a whole row to one wave).  Arithmetic as above: the max over the row's
-// scores; run_mh: den = the sum in position order of libm expf(s - max) (one thread, chunk by
+// output of a pass of few rows (a verify pass or short block, M <= 8): one block per (row, head), one
+// output dim per thread, so that every dim's chain over the positions has a thread of its own.
+// The max over the row's scores; run_mh: den = the sum in position order of libm expf(s - max) (one thread, chunk by
 // chunk), w = expf(s - max) / den, out = r16(fma chain of w v in position order); attn_tile:
 // w = exp8(s - max), out = r16(chain * (1 / den)) with den the sum of w in order.  Weights are
 // staged per chunk of PF_RC positions from the 8-aligned position at or below lo, 0 where not
@@ -522,7 +365,7 @@ __global__ __launch_bounds__(D) void k_pf_attn_rows(const float* __restrict__ S,
 // a = r16(rms(x, pre_ff))
 __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_attn(const float* __restrict__ o, float* __restrict__ x,
                                                               float* __restrict__ a, const float* __restrict__ w1,
-                                                              const float* __restrict__ w2) {
+                                                              const float* __restrict__ w2, A8Rows aq) {
   __shared__ __align__(16) float os[H];
   __shared__ __align__(16) float xs[H];
   __shared__ double red[16];
@@ -562,7 +405,8 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_ff(const float* __restr
                                                             float* __restrict__ a, const float* __restrict__ w1,
                                                             const float* __restrict__ next_in_ln,
                                                             const float* __restrict__ fnorm, float scalar,
-                                                            float* __restrict__ h, int hrow, float* __restrict__ hn) {
+                                                            float* __restrict__ h, int hrow, float* __restrict__ hn,
+                                                            A8Rows aq) {
   __shared__ __align__(16) float os[H];
   __shared__ __align__(16) float xs[H];
   __shared__ double red[16];
@@ -576,7 +420,13 @@ __global__ __launch_bounds__(ROW_THREADS) void k_pf_post_ff(const float* __restr
     xs[i] = v;
     x[(size_t)m * H + i] = v;
   }
-  if (!next_in_ln && (hrow < 0 || m < hrow)) return;  // uniform
+  if (!next_in_ln && (hrow < 0 || m < hrow)) {  // uniform
+    if (aq.q) {  // the product that follows takes x itself
+      __syncthreads();
+      a8_store_row(aq, m, xs);
+    }
+    return;
+  }
   __syncthreads();
   const float r2 = block_rms_inv<H>(xs, red);
   if (next_in_ln && aq.q) {
@@ -631,8 +481,8 @@ __global__ void k_gm_pg_act(const float* __restrict__ pgv, const float* __restri
 }  // namespace
 
 void launch_pf_embed(const uint16_t* E, const int* toks, const float* in_ln, float sqh, float* x, float* a, int M,
-                     hipStream_t st) {
-  hipLaunchKernelGGL(k_pf_embed, dim3(M), dim3(ROW_THREADS), 0, st, E, toks, in_ln, sqh, x, a);
+                     hipStream_t st, const A8Rows& aq) {
+  hipLaunchKernelGGL(k_pf_embed, dim3(M), dim3(ROW_THREADS), 0, st, E, toks, in_ln, sqh, x, a, aq);
 }
 void launch_pf_qkv(float* q, const float* k, const float* v, const float* qn, const float* kn, const float* cs,
                    const float* sn, uint16_t* KC, uint16_t* VC, int P0, int M, hipStream_t st, int sib, int hd,
@@ -642,14 +492,18 @@ void launch_pf_qkv(float* q, const float* k, const float* v, const float* qn, co
   else
     hipLaunchKernelGGL(k_pf_qkv<HD>, dim3(M), dim3(HD), 0, st, q, k, v, qn, kn, cs, sn, KC, VC, P0, sib, own, dpos);
 }
-long long pf_score_floats(int M, int Pb, int sliding) {
-  const long long R = M;
-  if (!sliding) return 8 * (R * (Pb + 1) + R * (R - 1) / 2);
-  const long long c = std::min<long long>(std::max(512 - Pb, 0), R);
-  return 8 * (c * (Pb + 1) + c * (c - 1) / 2 + (R - c) * 512);
+// (either layer type; up to M rows)
+long long pf_score_floats(int M, int Pb) {
+  const long long R = std::min(M, MAXM), few = 8 * (R * (Pb + 1 + M - R) + R * (R - 1) / 2);
+  return M > MAXM ? std::max(few, pfa_scratch_floats(M, Pb)) : few;
 }
 void launch_pf_attn(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g,
-                    int r0, int M, int sliding, hipStream_t st, bool staged, int hd, const int* dpos, int maxpos) {
+                    int r0, int M, int sliding, hipStream_t st, bool staged, int hd, const int* dpos, int maxpos,
+                    const A8Rows& aq) {
+  if (M > MAXM) {  // a prompt's rows: the matrix-core kernels (no sibling, position from the host, plain rows)
+    launch_pfa(q, KC, VC, S, att, g, r0, M, sliding, st, hd, aq);
+    return;
+  }
   // (dpos: the position comes from device memory; the grid then covers positions below maxpos,
   // and the score blocks past a row's range return at once)
   const int Plast = dpos ? maxpos - 1 : g.pos0 + r0 + M - 1;
@@ -657,36 +511,29 @@ void launch_pf_attn(const float* q, const uint16_t* KC, const uint16_t* VC, floa
   const int maxlen = sliding ? std::min(Plast + 1, g.sib >= 0 ? r0 + M - 1 + 511 : 512) : Plast + 1;
   const int spans = (maxlen + PF_SPAN - 1) / PF_SPAN;
   ExpfTab tab{G4V_EXPF_TABLE};
-  // a pass of few rows gives every (row, head) a block; a prompt block keeps a wave per row (it
-  // reads each value row once for the 8 heads)
-  const bool rows = M <= MAXM;
   if (hd == 512) {
     hipLaunchKernelGGL(k_pf_scores<512>, dim3(M, spans), dim3(256), 0, st, q, KC, S, g, r0, sliding, dpos);
-    if (rows)
-      hipLaunchKernelGGL(k_pf_attn_rows<512>, dim3(M, NQ), dim3(512), 0, st, S, VC, att, g, r0, sliding, tab,
-                         staged ? 1 : 0, dpos);
-    else
-      hipLaunchKernelGGL(k_pf_attn_out<512>, dim3(M), dim3(64), 0, st, S, VC, att, g, r0, sliding, tab, staged ? 1 : 0, dpos);
+    hipLaunchKernelGGL(k_pf_attn_rows<512>, dim3(M, NQ), dim3(512), 0, st, S, VC, att, g, r0, sliding, tab,
+                       staged ? 1 : 0, dpos);
   } else {
     hipLaunchKernelGGL(k_pf_scores<HD>, dim3(M, spans), dim3(256), 0, st, q, KC, S, g, r0, sliding, dpos);
-    if (rows)
-      hipLaunchKernelGGL(k_pf_attn_rows<HD>, dim3(M, NQ), dim3(HD), 0, st, S, VC, att, g, r0, sliding, tab,
-                         staged ? 1 : 0, dpos);
-    else
-      hipLaunchKernelGGL(k_pf_attn_out<HD>, dim3(M), dim3(64), 0, st, S, VC, att, g, r0, sliding, tab, staged ? 1 : 0, dpos);
+    hipLaunchKernelGGL(k_pf_attn_rows<HD>, dim3(M, NQ), dim3(HD), 0, st, S, VC, att, g, r0, sliding, tab,
+                       staged ? 1 : 0, dpos);
   }
 }
-void launch_pf_post_attn(const float* o, float* x, float* a, const float* w1, const float* w2, int M, hipStream_t st) {
-  hipLaunchKernelGGL(k_pf_post_attn, dim3(M), dim3(ROW_THREADS), 0, st, o, x, a, w1, w2);
+void launch_pf_post_attn(const float* o, float* x, float* a, const float* w1, const float* w2, int M, hipStream_t st,
+                         const A8Rows& aq) {
+  hipLaunchKernelGGL(k_pf_post_attn, dim3(M), dim3(ROW_THREADS), 0, st, o, x, a, w1, w2, aq);
 }
 void launch_pf_act(const float* g, const float* u, float* act, size_t n, hipStream_t st) {
   const int grid = (int)std::min<size_t>((n + 255) / 256, 8192);
   hipLaunchKernelGGL(k_pf_act, dim3(grid), dim3(256), 0, st, g, u, act, n);
 }
 void launch_pf_post_ff(const float* o, float* x, float* a, const float* w1, const float* next_in_ln,
-                       const float* fnorm, float scalar, float* h, int hrow, int M, hipStream_t st, float* hn) {
+                       const float* fnorm, float scalar, float* h, int hrow, int M, hipStream_t st, float* hn,
+                       const A8Rows& aq) {
   hipLaunchKernelGGL(k_pf_post_ff, dim3(M), dim3(ROW_THREADS), 0, st, o, x, a, w1, next_in_ln, fnorm, scalar, h,
-                     hrow, hn);
+                     hrow, hn, aq);
 }
 void launch_gm_ple(const float* pr, const int* toks, const uint16_t* ple, const float* plnorm, float* pli, int M,
                    hipStream_t st) {

@@ -28,10 +28,10 @@ namespace g4v {
 
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8_t;
 typedef __attribute__((ext_vector_type(4))) float f32x4_t;
+typedef __attribute__((ext_vector_type(4))) uint32_t u32x4_t;
 
-// within each 8-element k-slice the operands hold elements in the order 0,2,4,6,1,3,5,7
-// (low nibbles first, then high nibbles), which keeps the weight decode to byte permutes
-__host__ __device__ constexpr int a8_slot_elem(int j) { return j < 4 ? 2 * j : 2 * (j - 4) + 1; }
+// within each 8-element k-slice the operands hold elements in the order 0,2,4,6,1,3,5,7 (a8_slot: low
+// nibbles first, then high nibbles), which keeps the weight decode to byte permutes
 
 // orig w [N][K/2] (low nibble = even k), s [N][K/32] bf16  ->
 // tw [N/16][G/4][64] uint4, ts [N/16][G/8][16] uint4 (8 scales of one row)
@@ -64,75 +64,46 @@ void launch_tile_a8(const uint8_t* w, const uint16_t* s, uint4* tw, uint4* ts, i
   hipLaunchKernelGGL(k_tile_a8, dim3(grid), dim3(256), 0, st, w, s, tw, ts, N, K);
 }
 
-// A8:30-42 per (row m, group g); rows M .. Mpad-1 are written as zeros (the MFMA reads them).
-// xqb [Mpad][K] bf16 in the slot order; sxt / corr [G][Mpad]; optional q [M][K] int8 (plain
+// A8:30-42: a thread takes 8 consecutive values, four neighbouring lanes a group (with a thread per
+// group the lanes' 128-byte rows cost 78 us for 6,841 x 6,144 values).  Optional q [M][K] int8 (plain
 // order), sx / sum [M][G] for the quant entry point.
-__global__ void k_w4a8_quant(const float* __restrict__ x, int M, int Mpad, int K, uint16_t* __restrict__ xqb,
-                             float* __restrict__ sxt, float* __restrict__ corr, int8_t* __restrict__ qo,
-                             float* __restrict__ sxo, int32_t* __restrict__ sumo) {
-  const int G = K / 32;
-  const int idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= Mpad * G) return;
-  const int m = idx / G, g = idx - m * G;
-  uint4* dst = reinterpret_cast<uint4*>(xqb + (size_t)m * K + 32 * g);
-  if (m >= M) {
+__global__ __launch_bounds__(256) void k_w4a8_quant(const float* __restrict__ x, int M, int K, A8Rows o,
+                                                    int8_t* __restrict__ qo, float* __restrict__ sxo,
+                                                    int32_t* __restrict__ sumo) {
+  const size_t u = (size_t)blockIdx.x * 256 + threadIdx.x;
+  const int K8 = K / 8;
+  if (u >= (size_t)M * K8) return;  // whole groups: M K / 8 is a multiple of 4
+  const int m = (int)(u / K8), i = (int)(u - (size_t)m * K8);
+  const float4 a = *reinterpret_cast<const float4*>(x + 8 * u), b = *reinterpret_cast<const float4*>(x + 8 * u + 4);
+  const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+  a8_store8(o, m, K, i, v);
+  if (qo) {  // (uniform)
+    float amax = 0.f, sum = 0.f, q[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) dst[i] = make_uint4(0, 0, 0, 0);
-    sxt[(size_t)g * Mpad + m] = 0.f;
-    corr[(size_t)g * Mpad + m] = 0.f;
-    return;
-  }
-  const float4* p = reinterpret_cast<const float4*>(x + (size_t)m * K + 32 * g);
-  float v[32];
+    for (int k = 0; k < 8; ++k) amax = fmaxf(amax, fabsf(v[k]));
+    amax = fmaxf(amax, dpp_f(amax, 2));
+    amax = fmaxf(amax, dpp_f(amax, 3));
+    const float sx = amax / 127.0f, inv = sx > 0.f ? 1.0f / sx : 0.0f;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const float4 f = p[i];
-    v[4 * i] = f.x;
-    v[4 * i + 1] = f.y;
-    v[4 * i + 2] = f.z;
-    v[4 * i + 3] = f.w;
-  }
-  float amax = 0.f;
+    for (int k = 0; k < 8; ++k) q[k] = a8_q(v[k], inv, sum);
+    sum += dpp_f(sum, 2);
+    sum += dpp_f(sum, 3);
+    uint32_t w[2] = {0, 0};
 #pragma unroll
-  for (int i = 0; i < 32; ++i) amax = fmaxf(amax, fabsf(v[i]));
-  const float sx = amax / 127.0f, inv = sx > 0.f ? 1.0f / sx : 0.0f;
-  int q[32];
-  int sum = 0;
-#pragma unroll
-  for (int i = 0; i < 32; ++i) {
-    q[i] = (int)__builtin_rintf(v[i] * inv);  // RNE, as _mm256_cvtps_epi32 in the default mode
-    sum += q[i];
-    q[i] = q[i] > 127 ? 127 : (q[i] < -128 ? -128 : q[i]);
-  }
-  uint32_t packed[16];
-#pragma unroll
-  for (int sl = 0; sl < 4; ++sl)
-#pragma unroll
-    for (int j = 0; j < 8; j += 2) {
-      const uint32_t b0 = as_u32((float)q[8 * sl + a8_slot_elem(j)]) >> 16;
-      const uint32_t b1 = as_u32((float)q[8 * sl + a8_slot_elem(j + 1)]) >> 16;
-      packed[sl * 4 + j / 2] = b0 | (b1 << 16);
+    for (int k = 0; k < 8; ++k) w[k >> 2] |= ((uint32_t)(int)q[k] & 0xFFu) << (8 * (k & 3));
+    *reinterpret_cast<uint2*>(qo + 8 * u) = make_uint2(w[0], w[1]);
+    if ((i & 3) == 0) {
+      sxo[u >> 2] = sx;
+      sumo[u >> 2] = (int32_t)sum;
     }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) dst[i] = make_uint4(packed[4 * i], packed[4 * i + 1], packed[4 * i + 2], packed[4 * i + 3]);
-  sxt[(size_t)g * Mpad + m] = sx;
-  corr[(size_t)g * Mpad + m] = (float)(-136 * sum);
-  if (qo) {
-    uint32_t* qd = reinterpret_cast<uint32_t*>(qo + (size_t)m * K + 32 * g);
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      qd[i] = (uint32_t)(q[4 * i] & 0xFF) | ((uint32_t)(q[4 * i + 1] & 0xFF) << 8) |
-              ((uint32_t)(q[4 * i + 2] & 0xFF) << 16) | ((uint32_t)(q[4 * i + 3] & 0xFF) << 24);
-    sxo[(size_t)m * G + g] = sx;
-    sumo[(size_t)m * G + g] = sum;
   }
 }
 
 void launch_w4a8_quant(const float* x, int M, int Mpad, int K, uint16_t* xqb, float* sxt, float* corr, int8_t* qo,
                        float* sxo, int32_t* sumo, hipStream_t st) {
-  const int n = Mpad * (K / 32);
-  hipLaunchKernelGGL(k_w4a8_quant, dim3((n + 127) / 128), dim3(128), 0, st, x, M, Mpad, K, xqb, sxt, corr, qo, sxo,
-                     sumo);
+  const size_t n = (size_t)M * (K / 8);
+  hipLaunchKernelGGL(k_w4a8_quant, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, x, M, K,
+                     A8Rows{xqb, sxt, corr, Mpad}, qo, sxo, sumo);
 }
 
 // bf16(128 + u) for the four low (sel 0x04010400 / 0x04030402 of the lo word) or high nibbles
@@ -146,188 +117,283 @@ __device__ __forceinline__ bf16x8_t a8_decode(uint32_t d) {
   return __builtin_bit_cast(bf16x8_t, o);
 }
 
-// One wave per 16 output columns (tile t) and MT m-tiles of 16 rows (rows m0 .. m0 + 16 MT - 1).
-// Lane (r, h): B column r, A row r, k-slice h; D element i = row 4h + i, column r.
-template <int MT>
-__global__ __launch_bounds__(256) void k_w4a8_gemm(const uint4* __restrict__ tw, const uint4* __restrict__ ts,
-                                                   const uint16_t* __restrict__ xqb, const float* __restrict__ sxt,
-                                                   const float* __restrict__ corr, float* __restrict__ y, int M,
-                                                   int Mpad, int N, int K, int ldy) {
-  const int lane = threadIdx.x & 63;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-  if (t >= N / 16) return;  // whole waves; the kernel has no block-level barrier
-  const int m0 = blockIdx.y * 16 * MT;
+// Products of more than 8 rows.  A block of 4 waves covers 16 MT rows and 4 NT tiles of 16 outputs
+// (wave w the tiles NT w ..); lane (r, h): B column r, A row r, k-slice h; D element i = row 4h + i,
+// column r.  The block's operand rows, corrections and row scales of a step of CG groups are loaded
+// once per block a step ahead into registers and written to the other half of a double-buffered
+// LDS stage, one LDS barrier per step (the weights, each wave's own, stay in flight across it).
+// PAIR: the NT tiles are NT / 2 gate tiles (matrix 0) and the same outputs' up tiles (matrix 1), and
+// the activation r16(r16(gelu8(r16 g)) * r16 u) leaves as down's quantised rows (A8Gemm::yq).
+template <int MT, int NT, int CG, bool PAIR>
+__global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm q, const uint16_t* __restrict__ xqb,
+                                                   const float* __restrict__ sxt, const float* __restrict__ corr,
+                                                   int M, int Mpad, int K) {
+  constexpr int RB = 16 * MT, ROWB = CG * 64 + 16;  // rows of a block, bytes of a staged row (+ pad)
+  constexpr int NP = MT * CG / 4;                   // 16-byte pieces per thread and step
+  constexpr int NC = CG * RB, NCT = (NC + 255) / 256;
+  static_assert(MT * CG % 4 == 0 && (CG == 4 || CG == 8), "whole pieces, whole chunks of 4 groups");
+  __shared__ __align__(16) uint8_t As[2][RB * ROWB];
+  __shared__ __align__(16) float Cs[2][CG][RB], Ss[2][CG][RB];
+  const int lane = threadIdx.x & 63, tid = threadIdx.x, w = threadIdx.x >> 6;
+  constexpr int TPW = PAIR ? NT / 2 : NT;           // tiles of a matrix per wave
+  const int tg = (blockIdx.x * 4 + w) * TPW;        // first of the wave's tiles over the matrices
+  const bool active = tg < q.t0[PAIR ? 1 : 3];      // idle waves still stage and wait
+  const int tw = active ? tg : 0;
+  const int mi = PAIR ? 0 : ((tw >= q.t0[1]) + (tw >= q.t0[2]));
+  const int t0 = tw - (mi == 0 ? 0 : (mi == 1 ? q.t0[1] : q.t0[2]));
+  const int m0 = blockIdx.y * RB;
   const int r = lane & 15, h = lane >> 4;
-  const int G = K / 32;
-  const uint4* wp = tw + (size_t)t * (G / 4) * 64 + lane;  // chunk c at + 64 c
-  const uint4* sp = ts + (size_t)t * (G / 8) * 16 + r;     // scales of groups 8 c8 .. at + 16 c8
-  const uint16_t* ap = xqb + (size_t)(m0 + r) * K + 8 * h;  // m-tile mt, group g at + 16 mt K + 32 g
-  const int mrow = m0 + 4 * h;                              // + 16 mt: first D row of the lane
-  float acc[MT][4];
+  const int G = K / 32, NS = G / CG;
+  const uint4 *wp[NT], *sp[NT];  // chunk c of 4 groups at wp + 64 c, scales of 8 groups at sp + 16 c8
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) acc[mt][i] = 0.f;
-
-  uint4 wv = wp[0], sv = sp[0];
-  for (int c = 0; c < G / 4; ++c) {
-    const uint4 wcur = wv, scur = sv;
-    if (c + 1 < G / 4) wv = wp[(size_t)(c + 1) * 64];
-    if ((c & 1) && c + 1 < G / 4) sv = sp[(size_t)((c + 1) >> 1) * 16];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int g = 4 * c + i;
-      const uint32_t d = i == 0 ? wcur.x : (i == 1 ? wcur.y : (i == 2 ? wcur.z : wcur.w));
-      const bf16x8_t B = a8_decode(d);
-      const int gi = 4 * (c & 1) + i;  // group within the 8 scales of scur
-      const uint32_t s2 = gi < 2 ? scur.x : (gi < 4 ? scur.y : (gi < 6 ? scur.z : scur.w));
-      const float sw = as_f32((gi & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
-#pragma unroll
-      for (int mt = 0; mt < MT; ++mt) {
-        const uint4 av = *reinterpret_cast<const uint4*>(ap + (size_t)mt * 16 * K + 32 * g);
-        const float4 cr = *reinterpret_cast<const float4*>(corr + (size_t)g * Mpad + mrow + 16 * mt);
-        const float4 sx = *reinterpret_cast<const float4*>(sxt + (size_t)g * Mpad + mrow + 16 * mt);
-        const f32x4_t cin = {cr.x, cr.y, cr.z, cr.w};
-        const f32x4_t a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, av), B, cin, 0, 0, 0);
-        acc[mt][0] = fmaf(a[0], sw * sx.x, acc[mt][0]);  // A8:59 sc = sw * sx, row = fma(a32, sc, row)
-        acc[mt][1] = fmaf(a[1], sw * sx.y, acc[mt][1]);
-        acc[mt][2] = fmaf(a[2], sw * sx.z, acc[mt][2]);
-        acc[mt][3] = fmaf(a[3], sw * sx.w, acc[mt][3]);
-      }
+  for (int u = 0; u < NT; ++u) {
+    const int t = t0 + (PAIR ? u % TPW : u);
+    const uint4 *tww = q.tw[0], *tss = q.ts[0];
+    if constexpr (PAIR) {
+      if (u >= TPW) tww = q.tw[1], tss = q.ts[1];
+    } else {
+      if (mi == 1) tww = q.tw[1], tss = q.ts[1];
+      if (mi == 2) tww = q.tw[2], tss = q.ts[2];
     }
+    wp[u] = tww + (size_t)t * (G / 4) * 64 + lane;
+    sp[u] = tss + (size_t)t * (G / 8) * 16 + r;
   }
+  f32x4_t acc[MT][NT];
 #pragma unroll
   for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int m = mrow + 16 * mt + i;
-      if (m < M) y[(size_t)m * ldy + 16 * t + r] = acc[mt][i];
+    for (int u = 0; u < NT; ++u) acc[mt][u] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+  u32x4_t ap[NP];
+  float crn[NCT], sxn[NCT];
+  auto issue = [&](int st) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const int i = tid + 256 * k;  // row i / (4 CG), 16 bytes i % (4 CG) of the step
+      ap[k] = *reinterpret_cast<const u32x4_t*>(xqb + (size_t)(m0 + i / (4 * CG)) * K + 32 * CG * st + 8 * (i % (4 * CG)));
     }
-}
-
-// LDS-staged variant for long M (prefill): a block of 4 waves covers 64 rows (MT = 4 m-tiles)
-// and 4 x NT 16-column tiles (NT = 2: 145 VGPRs, 3 waves per SIMD).  The block's activation fragments, corrections and row scales of
-// a chunk of 4 groups are loaded once per block (not once per wave) a chunk ahead into
-// registers, then written to the other half of a double-buffered LDS stage; one barrier per
-// chunk.  Same arithmetic, in the same order, as k_w4a8_gemm.
-constexpr int A8_ROWB = 128 * 2 + 16;  // bytes of one staged row: 4 groups x 32 bf16, + pad
-template <int NT>
-__global__ __launch_bounds__(256) void k_w4a8_gemm_lds(const uint4* __restrict__ tw, const uint4* __restrict__ ts,
-                                                       const uint16_t* __restrict__ xqb, const float* __restrict__ sxt,
-                                                       const float* __restrict__ corr, float* __restrict__ y, int M,
-                                                       int Mpad, int N, int K, int ldy) {
-  constexpr int MT = 4;
-  __shared__ __align__(16) uint8_t As[2][64 * A8_ROWB];
-  __shared__ __align__(16) float Cs[2][4][64], Ss[2][4][64];
-  const int lane = threadIdx.x & 63, tid = threadIdx.x;
-  const int t0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * NT;  // first 16-column tile of the wave
-  const bool active = t0 < N / 16;                            // idle waves still stage and wait
-  const int m0 = blockIdx.y * 64;
-  const int r = lane & 15, h = lane >> 4;
-  const int G = K / 32, NC = G / 4;
-  const int tt0 = active ? t0 : 0;
-  const uint4* wp = tw + (size_t)tt0 * (G / 4) * 64 + lane;
-  const uint4* sp = ts + (size_t)tt0 * (G / 8) * 16 + r;
-  // staging roles: thread tid loads 16-byte pieces tid, tid + 256, tid + 512, tid + 768 of the
-  // 64 x 256-byte chunk (row = piece / 16, column piece % 16), i.e. column tid % 16 of rows
-  // tid / 16 + 16 k, and entry tid of the 4 x 64 corrections / scales
-  const int sg = tid >> 6, sm = tid & 63;
-  const uint16_t* arow = xqb + (size_t)(m0 + (tid >> 4)) * K + 8 * (tid & 15);  // piece tid; + 16 rows per k
-  const int aoff = (tid >> 4) * A8_ROWB + 16 * (tid & 15);
-  float acc[MT][NT][4];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+    for (int k = 0; k < NCT; ++k) {
+      const int i = (tid + 256 * k) & (NC - 1), g = i / RB, m = i % RB;
+      crn[k] = corr[(size_t)(CG * st + g) * Mpad + m0 + m];
+      sxn[k] = sxt[(size_t)(CG * st + g) * Mpad + m0 + m];
+    }
+  };
+  auto commit = [&](int b) {
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+      const int i = tid + 256 * k;
+      *reinterpret_cast<u32x4_t*>(&As[b][(i / (4 * CG)) * ROWB + 16 * (i % (4 * CG))]) = ap[k];
+    }
+#pragma unroll
+    for (int k = 0; k < NCT; ++k) {  // (with fewer than 256 entries several threads store the same)
+      const int i = (tid + 256 * k) & (NC - 1);
+      Cs[b][i / RB][i % RB] = crn[k];
+      Ss[b][i / RB][i % RB] = sxn[k];
+    }
+  };
+  static_assert((NC & (NC - 1)) == 0, "a power of two of corrections");
+  // weight words (chunks of 4 groups) of the current and the next step in two register sets that swap
+  // roles, the 8 scales of a row likewise (one word serves a step of 8 groups, or two of 4)
+  constexpr int CW = CG / 4;
+  u32x4_t wA[NT][CW], wB[NT][CW], sA[NT], sB[NT];
+  auto issue_w = [&](u32x4_t (&wx)[NT][CW], int st) {
 #pragma unroll
     for (int u = 0; u < NT; ++u)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc[mt][u][i] = 0.f;
-  uint4 wv[NT], sv[NT];
+      for (int k = 0; k < CW; ++k)
+        wx[u][k] = *reinterpret_cast<const u32x4_t*>(wp[u] + (size_t)(CW * st + k) * 64);
+  };
+  auto issue_s = [&](u32x4_t (&sx)[NT], int c8) {
 #pragma unroll
-  for (int u = 0; u < NT; ++u) {
-    wv[u] = wp[(size_t)u * (G / 4) * 64];
-    sv[u] = sp[(size_t)u * (G / 8) * 16];
-  }
-  uint4 a0 = *reinterpret_cast<const uint4*>(arow), a1 = *reinterpret_cast<const uint4*>(arow + 16 * K),
-        a2 = *reinterpret_cast<const uint4*>(arow + 32 * K), a3 = *reinterpret_cast<const uint4*>(arow + 48 * K);
-  float crn = corr[(size_t)sg * Mpad + m0 + sm], sxn = sxt[(size_t)sg * Mpad + m0 + sm];
-  *reinterpret_cast<uint4*>(&As[0][aoff]) = a0;
-  *reinterpret_cast<uint4*>(&As[0][aoff + 16 * A8_ROWB]) = a1;
-  *reinterpret_cast<uint4*>(&As[0][aoff + 32 * A8_ROWB]) = a2;
-  *reinterpret_cast<uint4*>(&As[0][aoff + 48 * A8_ROWB]) = a3;
-  Cs[0][sg][sm] = crn;
-  Ss[0][sg][sm] = sxn;
-  __syncthreads();
-  for (int c = 0; c < NC; ++c) {
-    const int b = c & 1;
-    if (c + 1 < NC) {  // uniform: the next chunk's rows, corrections and scales
-      const uint16_t* an = arow + 128 * (c + 1);
-      a0 = *reinterpret_cast<const uint4*>(an);
-      a1 = *reinterpret_cast<const uint4*>(an + 16 * K);
-      a2 = *reinterpret_cast<const uint4*>(an + 32 * K);
-      a3 = *reinterpret_cast<const uint4*>(an + 48 * K);
-      crn = corr[(size_t)(4 * (c + 1) + sg) * Mpad + m0 + sm];
-      sxn = sxt[(size_t)(4 * (c + 1) + sg) * Mpad + m0 + sm];
-    }
-    uint4 wcur[NT], scur[NT];
+    for (int u = 0; u < NT; ++u) sx[u] = *reinterpret_cast<const u32x4_t*>(sp[u] + (size_t)c8 * 16);
+  };
+  auto products = [&](const int b, const u32x4_t (&wc)[NT][CW], const u32x4_t (&sc8)[NT]) {
 #pragma unroll
-    for (int u = 0; u < NT; ++u) {
-      wcur[u] = wv[u];
-      scur[u] = sv[u];
-      if (c + 1 < NC) wv[u] = wp[((size_t)u * (G / 4) + c + 1) * 64];
-      if ((c & 1) && c + 1 < NC) sv[u] = sp[((size_t)u * (G / 8) + ((c + 1) >> 1)) * 16];
-    }
-    if (active) {
+    for (int i = 0; i < CG; ++i) {
+      const int e = CG == 4 ? 4 * b + i : i;  // group within the 8 scales
+      bf16x8_t B[NT];
+      float sw[NT];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int gi = 4 * (c & 1) + i;
-        bf16x8_t B[NT];
-        float sw[NT];
+      for (int u = 0; u < NT; ++u) {
+        B[u] = a8_decode(wc[u][i >> 2][i & 3]);
+        const uint32_t s2 = sc8[u][e >> 1];
+        sw[u] = as_f32((e & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
+      }
+#pragma unroll
+      for (int mt = 0; mt < MT; ++mt) {
+        const u32x4_t av = *reinterpret_cast<const u32x4_t*>(&As[b][(16 * mt + r) * ROWB + 64 * i + 16 * h]);
+        const f32x4_t cin = *reinterpret_cast<const f32x4_t*>(&Cs[b][i][16 * mt + 4 * h]);
+        const f32x4_t sx = *reinterpret_cast<const f32x4_t*>(&Ss[b][i][16 * mt + 4 * h]);
+        const bf16x8_t A = __builtin_bit_cast(bf16x8_t, av);
 #pragma unroll
         for (int u = 0; u < NT; ++u) {
-          const uint32_t d = i == 0 ? wcur[u].x : (i == 1 ? wcur[u].y : (i == 2 ? wcur[u].z : wcur[u].w));
-          B[u] = a8_decode(d);
-          const uint32_t s2 = gi < 2 ? scur[u].x : (gi < 4 ? scur[u].y : (gi < 6 ? scur[u].z : scur[u].w));
-          sw[u] = as_f32((gi & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
+          const f32x4_t a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[u], cin, 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) acc[mt][u][k] = fmaf(a[k], sw[u] * sx[k], acc[mt][u][k]);  // A8:59
         }
+      }
+    }
+  };
+  issue(0);
+  issue_w(wA, 0);
+  issue_s(sA, 0);
+  commit(0);
+  lds_barrier();
+  // (NS is even with steps of 4 groups: K % 256 == 0; with 8 it may be odd; the prefetch past the last
+  // step reads that step again and is not used)
+  for (int st = 0; st < NS; st += 2) {
+    issue(min(st + 1, NS - 1));
+    issue_w(wB, min(st + 1, NS - 1));
+    issue_s(sB, CG == 4 ? min(st / 2 + 1, NS / 2 - 1) : min(st + 1, NS - 1));
+    products(0, wA, sA);
+    commit(1);
+    lds_barrier();
+    if (CG == 8 && st + 1 >= NS) break;  // uniform
+    issue(min(st + 2, NS - 1));
+    issue_w(wA, min(st + 2, NS - 1));
+    if constexpr (CG == 4) {
+      products(1, wB, sA);
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-          const uint4 av = *reinterpret_cast<const uint4*>(&As[b][(16 * mt + r) * A8_ROWB + 64 * i + 16 * h]);
-          const float4 cr = *reinterpret_cast<const float4*>(&Cs[b][i][16 * mt + 4 * h]);
-          const float4 sx = *reinterpret_cast<const float4*>(&Ss[b][i][16 * mt + 4 * h]);
-          const f32x4_t cin = {cr.x, cr.y, cr.z, cr.w};
-          const bf16x8_t A = __builtin_bit_cast(bf16x8_t, av);
+      for (int u = 0; u < NT; ++u) sA[u] = sB[u];
+    } else {
+      issue_s(sA, min(st + 2, NS - 1));
+      products(1, wB, sB);
+    }
+    commit(0);
+    lds_barrier();
+  }
+  if (!active) return;
+  if constexpr (PAIR) {
+    // TPW = 2: the wave's two tiles are one 32-group of the activation, quantised here for down; the
+    // sixteen lanes r hold two of its values each
+    static_assert(TPW == 2, "a wave owns whole groups");
+    const int g = t0 >> 1;  // (t0 is even)
+    const int N = 16 * q.t0[1];
 #pragma unroll
-          for (int u = 0; u < NT; ++u) {
-            const f32x4_t a = __builtin_amdgcn_mfma_f32_16x16x32_bf16(A, B[u], cin, 0, 0, 0);
-            acc[mt][u][0] = fmaf(a[0], sw[u] * sx.x, acc[mt][u][0]);  // A8:59
-            acc[mt][u][1] = fmaf(a[1], sw[u] * sx.y, acc[mt][u][1]);
-            acc[mt][u][2] = fmaf(a[2], sw[u] * sx.z, acc[mt][u][2]);
-            acc[mt][u][3] = fmaf(a[3], sw[u] * sx.w, acc[mt][u][3]);
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int m = m0 + 16 * mt + 4 * h + i;
+        float v[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) v[u] = r16(r16(gelu8(r16(acc[mt][u][i]))) * r16(acc[mt][u + 2][i]));
+        const float amax = row16_all_max(fmaxf(fabsf(v[0]), fabsf(v[1])));
+        const float sx = amax / 127.0f, inv = sx > 0.f ? 1.0f / sx : 0.0f;
+        float sum = 0.f;
+        const float q0 = a8_q(v[0], inv, sum), q1 = a8_q(v[1], inv, sum);
+        sum = row16_all_sum(sum);
+        if (m < M) {
+          uint16_t* d = q.yq.q + (size_t)m * N + 32 * g + a8_slot(r);
+          d[0] = (uint16_t)(as_u32(q0) >> 16);
+          d[16] = (uint16_t)(as_u32(q1) >> 16);
+          if (r == 0) {
+            q.yq.sx[(size_t)g * q.yq.ld + m] = sx;
+            q.yq.corr[(size_t)g * q.yq.ld + m] = -136.0f * sum;
           }
         }
       }
-    }
-    if (c + 1 < NC) {  // the other half: last read before the previous barrier
-      *reinterpret_cast<uint4*>(&As[b ^ 1][aoff]) = a0;
-      *reinterpret_cast<uint4*>(&As[b ^ 1][aoff + 16 * A8_ROWB]) = a1;
-      *reinterpret_cast<uint4*>(&As[b ^ 1][aoff + 32 * A8_ROWB]) = a2;
-      *reinterpret_cast<uint4*>(&As[b ^ 1][aoff + 48 * A8_ROWB]) = a3;
-      Cs[b ^ 1][sg][sm] = crn;
-      Ss[b ^ 1][sg][sm] = sxn;
-    }
-    __syncthreads();
+  } else {
+    float* y = mi == 0 ? q.y[0] : (mi == 1 ? q.y[1] : q.y[2]);
+    const int ldy = mi == 0 ? q.ldy[0] : (mi == 1 ? q.ldy[1] : q.ldy[2]);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+      for (int u = 0; u < NT; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const int m = m0 + 16 * mt + 4 * h + i;
+          if (m < M) y[(size_t)m * ldy + 16 * (t0 + u) + r] = acc[mt][u][i];
+        }
   }
-  if (!active) return;
-  const int mrow = m0 + 4 * h;
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int u = 0; u < NT; ++u)
+}
+
+// The same products where they leave SIMDs idle (few tiles of 16 x 16): a block of eight waves per
+// tile.  Only the chain over the groups is ordered, so waves 0..3 form a phase's 16 group dots and
+// factors sw * sx (a chunk of 4 groups each, operands loaded two phases ahead) into LDS while waves
+// 4..7 run the previous phase's chains, D element i of every lane on wave 4 + i.  A lone wave issues an
+// instruction every ~6 cycles, and in k_w4a8_gemm's loop a tile's group took it ~300 cycles (40 rows,
+// K = 6144: 24 us on 288 waves); here a phase costs its four groups of dots.
+constexpr int SP_G = 16;  // groups of a phase
+__global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __restrict__ xqb,
+                                                    const float* __restrict__ sxt, const float* __restrict__ corr,
+                                                    int M, int Mpad, int K) {
+  __shared__ __align__(16) float2 S[2][SP_G][4][64];  // (a32, sw * sx) of D element i, lane
+  const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int tg = blockIdx.x, mi = (tg >= q.t0[1]) + (tg >= q.t0[2]);
+  const int t = tg - (mi == 0 ? 0 : (mi == 1 ? q.t0[1] : q.t0[2]));
+  const int m0 = blockIdx.y * 16, r = lane & 15, h = lane >> 4;
+  const int G = K / 32, NC = G / 4, NPH = (G + SP_G - 1) / SP_G;
+  const uint4 *tww = q.tw[0], *tss = q.ts[0];
+  if (mi == 1) tww = q.tw[1], tss = q.ts[1];
+  if (mi == 2) tww = q.tw[2], tss = q.ts[2];
+  if (w < 4) {
+    const uint4* wp = tww + (size_t)t * NC * 64 + lane;
+    const uint4* sp = tss + (size_t)t * (G / 8) * 16 + r;
+    const uint16_t* ap = xqb + (size_t)(m0 + r) * K + 8 * h;
+    const float *cp = corr + m0 + 4 * h, *xp = sxt + m0 + 4 * h;
+    struct Ops {
+      u32x4_t w, s, a[4];
+      f32x4_t c[4], x[4];
+    };
+    auto load = [&](Ops& o, int p) {  // chunk 4 p + w (past the last: that one again, not stored)
+      const int c = min(4 * p + w, NC - 1);
+      o.w = *reinterpret_cast<const u32x4_t*>(wp + (size_t)c * 64);
+      o.s = *reinterpret_cast<const u32x4_t*>(sp + (size_t)(c >> 1) * 16);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int m = mrow + 16 * mt + i;
-        if (m < M) y[(size_t)m * ldy + 16 * (t0 + u) + r] = acc[mt][u][i];
+        const size_t g = 4 * c + i;
+        o.a[i] = *reinterpret_cast<const u32x4_t*>(ap + 32 * g);
+        o.c[i] = *reinterpret_cast<const f32x4_t*>(cp + g * Mpad);
+        o.x[i] = *reinterpret_cast<const f32x4_t*>(xp + g * Mpad);
       }
+    };
+    auto form = [&](const Ops& o, int p) {
+      const int c = 4 * p + w;
+      if (c < NC) {  // uniform
+        const bool hi = c & 1;
+        const uint32_t s01 = hi ? o.s[2] : o.s[0], s23 = hi ? o.s[3] : o.s[1];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const uint32_t s2 = i < 2 ? s01 : s23;
+          const float sw = as_f32((i & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
+          const f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, o.a[i]),
+                                                                   a8_decode(o.w[i]), o.c[i], 0, 0, 0);
+#pragma unroll
+          for (int k = 0; k < 4; ++k) S[p & 1][4 * w + i][k][lane] = make_float2(d[k], sw * o.x[i][k]);
+        }
+      }
+      lds_barrier();
+    };
+    Ops A, B;
+    load(A, 0);
+    load(B, 1);
+    for (int p = 0; p < NPH; p += 2) {
+      form(A, p);
+      load(A, p + 2);
+      if (p + 1 < NPH) {  // uniform
+        form(B, p + 1);
+        load(B, p + 3);
+      }
+    }
+    return;
+  }
+  const int i = w - 4;
+  float acc = 0.f;
+  for (int p = 0; p < NPH; ++p) {
+    lds_barrier();  // phase p is formed; the producers go on to the other half
+    const float2* s = &S[p & 1][0][i][lane];
+    const int ng = min(SP_G, G - SP_G * p);  // 8 or 16: K % 256 == 0
+    for (int g8 = 0; g8 < ng; g8 += 8)
+#pragma unroll
+      for (int g = 0; g < 8; ++g) {
+        const float2 v = s[(g8 + g) * 256];
+        acc = fmaf(v.x, v.y, acc);  // A8:59
+      }
+  }
+  const int m = m0 + 4 * h + i;
+  float* y = mi == 0 ? q.y[0] : (mi == 1 ? q.y[1] : q.y[2]);
+  const int ldy = mi == 0 ? q.ldy[0] : (mi == 1 ? q.ldy[1] : q.ldy[2]);
+  if (m < M) y[(size_t)m * ldy + 16 * t + r] = acc;
 }
 
 // y [M][ldy] from the quantised rows; Mpad = M rounded up to 16 MT for the chosen MT
@@ -404,42 +470,61 @@ __global__ __launch_bounds__(1024) void k_w4a8_dec(A8Dec m, const uint16_t* __re
   if (tid < 128 && cm < M) y[(size_t)cm * ldy + 16 * t + cr] = acc;
 }
 
-int w4a8_mt(int M) { return M <= 16 ? 1 : (M <= 64 ? 2 : 4); }
-int w4a8_mpad(int M) {
-  const int bm = 16 * w4a8_mt(M);
+int w4a8_mpad(int M) {  // rows of the quantised operand: whole blocks of every shape used for M rows
+  const int bm = M <= 16 ? 16 : (M <= 64 ? 32 : 64);
   return (M + bm - 1) / bm * bm;
+}
+
+template <int MT, int NT, int CG, bool PAIR>
+static void launch_gemm(const A8Gemm& q, const uint16_t* xqb, const float* sxt, const float* corr, int M, int K,
+                        hipStream_t st) {
+  const int tpw = PAIR ? NT / 2 : NT, tiles = q.t0[PAIR ? 1 : 3];
+  const dim3 grid((tiles + 4 * tpw - 1) / (4 * tpw), (M + 16 * MT - 1) / (16 * MT));
+  hipLaunchKernelGGL((k_w4a8_gemm<MT, NT, CG, PAIR>), grid, dim3(256), 0, st, q, xqb, sxt, corr, M, w4a8_mpad(M), K);
+}
+
+int launch_w4a8_gemm_multi(const A8Gemm& q_in, int n, bool pair, const uint16_t* xqb, const float* sxt,
+                           const float* corr, int M, int K, hipStream_t st) {
+  A8Gemm q = q_in;
+  if (n < 1 || n > 3 || M < 1 || K % 256 || (pair && (n != 2 || q.N[0] != q.N[1] || q.N[0] % 32 || !q.yq.q))) return 0;
+  q.t0[0] = 0;
+  bool by4 = true;
+  int tiles = 0;
+  for (int j = 0; j < 3; ++j) {
+    if (j < n && q.N[j] % 16) return 0;
+    tiles += j < n ? q.N[j] / 16 : 0;
+    by4 = by4 && (j >= n || q.N[j] % 64 == 0);
+    q.t0[j + 1] = tiles;
+  }
+  if (pair) q.t0[1] = q.N[0] / 16;
+  const long waves1 = (long)tiles * ((M + 15) / 16);  // waves with a tile each
+  if (pair) {
+    if (by4 && M > 64 && waves1 > 8192) launch_gemm<4, 4, 4, true>(q, xqb, sxt, corr, M, K, st);
+    else launch_gemm<1, 4, 4, true>(q, xqb, sxt, corr, M, K, st);
+    return 1;
+  }
+  if (by4 && M > 64 && waves1 > 8192) launch_gemm<4, 4, 4, false>(q, xqb, sxt, corr, M, K, st);
+  else if (waves1 <= 1024)
+    hipLaunchKernelGGL(k_w4a8_split, dim3(tiles, (M + 15) / 16), dim3(512), 0, st, q, xqb, sxt, corr, M, w4a8_mpad(M), K);
+  else launch_gemm<1, 1, 8, false>(q, xqb, sxt, corr, M, K, st);
+  return 1;
 }
 
 void launch_w4a8_gemm(const uint4* tw, const uint4* ts, const uint16_t* xqb, const float* sxt, const float* corr,
                       float* y, int M, int N, int K, int ldy, hipStream_t st) {
-  const int MT = w4a8_mt(M), Mpad = w4a8_mpad(M);
-  if (M <= 8 && N % 16 == 0 && K % 256 == 0) {  // decode rows: group dots split over the block's waves
+  if (M <= 8) {  // decode rows: group dots split over the block's waves
     A8Dec m{};
     m.tw[0] = tw;
     m.ts[0] = ts;
     m.y[0] = y;
     m.ldy[0] = ldy;
     m.t0[1] = m.t0[2] = m.t0[3] = N / 16;
-    hipLaunchKernelGGL(k_w4a8_dec, dim3(N / 16), dim3(1024), 0, st, m, xqb, sxt, corr, M, Mpad, K);
+    hipLaunchKernelGGL(k_w4a8_dec, dim3(N / 16), dim3(1024), 0, st, m, xqb, sxt, corr, M, w4a8_mpad(M), K);
     return;
   }
-  if (MT == 4 && (N / 16) % 2 == 0 && K % 128 == 0) {  // long M: 4 x 2 tiles per wave, staged rows
-    const dim3 grid((N / 16 / 2 + 3) / 4, Mpad / 64);
-    hipLaunchKernelGGL(k_w4a8_gemm_lds<2>, grid, dim3(256), 0, st, tw, ts, xqb, sxt, corr, y, M, Mpad, N, K, ldy);
-    return;
-  }
-  const dim3 grid((N / 16 + 3) / 4, Mpad / (16 * MT));
-  switch (MT) {
-    case 1:
-      hipLaunchKernelGGL(k_w4a8_gemm<1>, grid, dim3(256), 0, st, tw, ts, xqb, sxt, corr, y, M, Mpad, N, K, ldy);
-      break;
-    case 2:
-      hipLaunchKernelGGL(k_w4a8_gemm<2>, grid, dim3(256), 0, st, tw, ts, xqb, sxt, corr, y, M, Mpad, N, K, ldy);
-      break;
-    default:
-      hipLaunchKernelGGL(k_w4a8_gemm<4>, grid, dim3(256), 0, st, tw, ts, xqb, sxt, corr, y, M, Mpad, N, K, ldy);
-      break;
-  }
+  A8Gemm q{};
+  q.tw[0] = tw, q.ts[0] = ts, q.y[0] = y, q.ldy[0] = ldy, q.N[0] = N;
+  (void)launch_w4a8_gemm_multi(q, 1, false, xqb, sxt, corr, M, K, st);
 }
 
 int launch_w4a8_dec(const A8Dec& m, int n, const uint16_t* xqb, const float* sxt, const float* corr, int M, int K,

@@ -103,6 +103,63 @@ def test_prefill_exact_float_row_tiles(orc, g4v, n, I):
         dev.close()
 
 
+# the many-row attention where row quads and key tiles end: the smallest pass (9 rows), blocks whose
+# path changes inside a quad (5 and 7 rows: run_mh up to position 64, attn_tile after), ranges that
+# start in a tile's middle (the 512 window), a global layer behind earlier context
+@pytest.mark.parametrize("n,NL,pfb,pos0", [(9, 1, 32, 0), (13, 2, 5, 58), (70, 1, 7, 0), (31, 1, 32, 33),
+                                           (45, 5, 32, 500), (33, 5, 16, 767)])
+def test_prefill_attention_tiles(orc, g4v, n, NL, pfb, pos0):
+    from oracle import Model
+    V, I, ctx, seed = 4096, 256, 1024, 23
+    toks = np.random.default_rng(n + pfb).integers(0, V, n).astype(np.int32)
+    note(f"prefill attention tiles n={n} NL={NL} pfb={pfb} pos0={pos0}")
+    dev = g4v.Device(0)
+    om = Model(orc, seed, V, NL, I, ctx)
+    try:
+        dev.model_synth(seed, V, NL, I, ctx)
+        if pos0:
+            dev.fake_ctx(pos0, 77)
+            om.fake_ctx(pos0, 77)
+        _, hd = dev.prefill(toks, pos0=pos0, pfb=pfb, hidden=True)
+        ho = om.prefill(toks, pos0=pos0, pfb=pfb)
+        assert same(hd, ho), first_diff(hd, ho)
+        for what in ("KC", "VC"):
+            a = dev.read(what, np.uint16).reshape(NL, -1, 256)[:, :pos0 + n]
+            b = om.get(what, np.uint16, NL * ctx * 256).reshape(NL, ctx, 256)[:, :pos0 + n]
+            assert same(a, b), (what, first_diff(a.ravel(), b.ravel()))
+    finally:
+        om.close()
+        dev.close()
+
+
+def test_prefill_attention_infinite_value(g4v):
+    """an infinite value at a position that only the first rows' windows hold: the later rows of the
+    same quad stay finite, bit for bit what passes of 8 rows (a thread per output dim) give"""
+    V, NL, I, ctx, pos0, n = 4096, 2, 256, 1024, 600, 24
+    toks = np.random.default_rng(4).integers(0, V, n).astype(np.int32)
+    note("prefill attention with an infinite value at the window's edge")
+    got = []
+    for parts in ((24,), (8, 8, 8)):
+        dev = g4v.Device(0)
+        try:
+            dev.model_synth(29, V, NL, I, ctx)
+            dev.set_prefill_int8(False)  # (the 8-bit rows of a NaN row are zeros)
+            dev.fake_ctx(pos0, 78)
+            k = np.full(256, 0x3C00, np.uint16)
+            v = np.full(256, 0x7F80, np.uint16)  # +inf; position 95 is in the windows of rows 600 .. 606
+            dev.set_kv(0, 95, k, v)
+            at = 0
+            for m in parts:
+                dev.prefill(toks[at:at + m], pos0=pos0 + at, pfb=8)
+                at += m
+            got.append(dev.read("KC", np.uint16).reshape(NL, -1, 256)[1, pos0:pos0 + n])
+        finally:
+            dev.close()
+    f = [(k.astype(np.uint32) << 16).view(np.float32) for k in got]  # layer 1's keys: layer 0's output
+    assert np.isnan(f[0][:7]).all() and np.isnan(f[1][:7]).all() and np.isfinite(f[0][7:]).all()
+    assert same(got[0][7:], got[1][7:])
+
+
 def test_prefill_then_lookup_decode(orc, g4v):
     """a motif prompt, then rounds of prompt-lookup drafts verified as a chain (E:1617-1661)"""
     from oracle import Model
