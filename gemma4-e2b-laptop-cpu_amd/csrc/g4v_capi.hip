@@ -1945,9 +1945,9 @@ static void pf_segment(g4v_ctx* c, const PfGeom& g, int r0, int M, bool i8, bool
                        NQ * HD, st);
     } else {
       launch_pf_attn(c->pfq.as<float>(), KCl, VCl, c->pfs.as<float>(), c->pfatt.as<float>(), g, r0, M, lay.sliding,
-                     st, false, HD, nullptr, 0, aq);
+                     st);
     }
-    pf_lin(c, lay.m[3], att, M, o, i8, false);  // E:1356
+    pf_lin(c, lay.m[3], att, M, o, i8, true);  // E:1356
     launch_pf_post_attn(o, x, a, ln.post_attn, ln.pre_ff, M, st, aq);
     pf_mlp(c, lay.m[4], lay.m[5], lay.m[6], a, M, gb, ub, act, o, i8);  // E:1366-1373
     const bool lastl = l + 1 == c->NL;
@@ -2132,10 +2132,10 @@ void gm_forward(g4v_ctx* c, int M, int pos0, int nsplit, int sib, int hrow, bool
                          NQ * HD, st);
     } else {  // attn_tile (M >= 4 past 64 keys, no sibling) or run_mh: one block of M rows
       launch_pf_attn(R.q, KCo, VCo, c->gm_s.as<float>(), R.att, pg ? *pg : PfGeom{M, pos0, M, sib}, 0, M, sliding,
-                     st, false, hd, dpos, c->ctxcap, aq);
+                     st, false, hd, dpos, c->ctxcap);
     }
     if (split) pmark(c, PT_ATTN, 0, 0);
-    pf_lin(c, lay.m[3], R.att, M, R.o, i8, false);                          // E:1356
+    pf_lin(c, lay.m[3], R.att, M, R.o, i8, true);                           // E:1356
     launch_pf_post_attn(R.o, R.x, R.a, post_attn, pre_ff, M, st, aq);       // E:1358-1361
     pf_mlp(c, lay.m[4], lay.m[5], lay.m[6], R.a, M, R.g, R.u, R.act, R.o, i8);  // E:1363-1373
     launch_pf_post_ff(R.o, R.x, R.a, post_ff, nullptr, nullptr, 1.0f, nullptr, -1, M, st, nullptr, aq);      // E:1375-1377

@@ -153,7 +153,7 @@ void launch_pf_qkv(float* q, const float* k, const float* v, const float* qn, co
 long long pf_score_floats(int M, int Pb);
 // attention of more than MAXM prompt rows (g4v_pfattn.hip), and its scratch
 void launch_pfa(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g, int r0,
-                int M, int sliding, hipStream_t st, int hd, const A8Rows& aq);
+                int M, int sliding, hipStream_t st, int hd);
 long long pfa_scratch_floats(int M, int Pb);
 // attn_tile / run_mh attention of segment rows [r0, r0 + M): q [n][2048] (row r at r), att likewise
 // staged: att rows in the staged GEMV input layout (staged_index) instead of plain.
@@ -161,7 +161,7 @@ long long pfa_scratch_floats(int M, int Pb);
 // run, so that a captured pass serves every position; the grid then covers positions below maxpos.
 void launch_pf_attn(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g,
                     int r0, int M, int sliding, hipStream_t st, bool staged = false, int hd = HD,
-                    const int* dpos = nullptr, int maxpos = 0, const A8Rows& aq = A8Rows{});
+                    const int* dpos = nullptr, int maxpos = 0);
 void launch_pf_post_attn(const float* o, float* x, float* a, const float* w1, const float* w2, int M, hipStream_t st,
                          const A8Rows& aq = A8Rows{});
 void launch_pf_act(const float* g, const float* u, float* act, size_t n, hipStream_t st);

@@ -1,19 +1,21 @@
 // g4v_pfattn.hip -- prompt attention (more than MAXM rows) on the fp32 matrix cores.
 //
 // The arithmetic of g4v_prefill.hip's attention (attn_tile E:1063-1083, run_mh E:1338-1349), chain
-// for chain.  v_mfma_f32_32x32x2_f32 adds its two products one after the other, each with one
-// rounding (the order and the roundings of fmaf, subnormals kept; g4v_gemmx.hip), so it runs the
-// reference's chains 32 x 32 at a time:
-//   scores: four chains of 2 prompt rows x 8 heads x 16 keys an instruction (k_pfa_scores);
-//     D / 32 instructions from 0 (attn_tile: steps tt = 2 i, 2 i + 1; run_mh: the one chain of lane l
-//     takes s = 0, 1 of step i), the lanes' sums meet in hsum's order;
-//   output: the same 32 rows, columns = 32 dims; O = fma(w, v, O) over the positions, two an
-//     instruction.
-// What bounds it: 66 cycles a SIMD per instruction of 2048 FMAs (31 FMAs a cycle; VALU fp32 work
-// reaches 22 and adds to it).  The VALU kernels this replaces read an LDS word per 1 (scores) or 4
-// (output) FMAs and reached half of the VALU rate.  Four rows a tile share every key and value word;
-// a block's waves split keys (scores) or dims (output), so no partial sums meet.
-// Measured, prompt of 6,841 rows (35 layers): scores 19.8 -> 13.3 ms, output 22.3 -> 12.1 ms.
+// for chain.  The fp32 matrix instructions add their products one after the other, each with one
+// rounding (the order and the roundings of fmaf, subnormals kept; g4v_gemmx.hip), so they run the
+// reference's chains 16 x 16 or 32 x 32 at a time:
+//   scores: v_mfma_f32_16x16x1_4b, four chains of 2 prompt rows x 8 heads x 16 keys an instruction
+//     (k_pfa_scores); the chains of a score meet in one lane, in hsum's order;
+//   output: v_mfma_f32_32x32x2, 4 prompt rows x 8 heads x 32 dims; O = fma(w, v, O) over the
+//     positions, two an instruction (k_pfa_out).
+// What bounds it: the matrix unit's 31 fp32 FMAs a cycle and SIMD (VALU fp32 work reaches 22 and adds
+// to it).  The VALU kernels this replaces read an LDS word per 1 (scores) or 4 (output) FMAs and
+// reached half of the VALU rate.  The rows of a tile share every key and value word; a block's waves
+// split rows (scores) or dims (output), so no partial sums meet.
+// Measured, prompt of 6,841 rows (28 window and 7 global layers): scores 19.8 -> 13.1 ms, output
+// 22.3 -> 11.9 ms.  The o product's input is quantised by a launch of its own: from the output's
+// registers (32 lanes a group) it cost 27 us a layer where that launch takes 22, and 9 for 3.5 at 40
+// rows.
 //
 // Scores go through memory as tiles [row quad][32 keys][32 rows x 32 keys] with each wave's row
 // maxima beside them: exp needs the row maximum first, and den the weights in position order.
@@ -199,7 +201,7 @@ __global__ __launch_bounds__(256, 2) void k_pfa_scores(const float* __restrict__
 template <int D>
 __global__ __launch_bounds__(D, 2) void k_pfa_out(const float* __restrict__ S, const float* __restrict__ PM,
                                                const uint16_t* __restrict__ VC, float* __restrict__ att, PfGeom g,
-                                               int r0, int M, int sliding, int nspan, A8Rows aq) {
+                                               int r0, int M, int sliding, int nspan) {
   constexpr int G8 = D / 32, CP = 8 * G8;  // groups of 8 positions, positions of a step
   __shared__ __align__(16) float W[2][G8][2][32][4];
   __shared__ uint64_t T[32];
@@ -373,29 +375,9 @@ __global__ __launch_bounds__(D, 2) void k_pfa_out(const float* __restrict__ S, c
     const bool tl = pfa_tiled(r0 + 4 * qd + t, g);
     const float ih = 1.0f / dens[m];
     const float v[2] = {tl ? r16(acc0[r] * ih) : r16(acc0[r]), tl ? r16(acc1[r] * ih) : r16(acc1[r])};
-    const int row = r0 + 4 * qd + t, n = (4 * half + (r & 3)) * D + 64 * w;  // dims n + c32, n + 32 + c32
-    if (!aq.q) {  // uniform
-      float* o = att + (size_t)row * NQ * D + n + c32;
-      o[0] = v[0];
-      o[32] = v[1];
-      continue;
-    }
-#pragma unroll
-    for (int u = 0; u < 2; ++u) {  // a 32-group of the o product's input on the half's 32 lanes
-      float amax = row16_all_max(fabsf(v[u]));
-      amax = fmaxf(amax, __shfl_xor(amax, 16));
-      const float sx = amax / 127.0f, inv = sx > 0.f ? 1.0f / sx : 0.0f;
-      float sum = 0.f;
-      const float qv = a8_q(v[u], inv, sum);
-      sum = row16_all_sum(sum);
-      sum += __shfl_xor(sum, 16);
-      const int gq = n / 32 + u, mq = row - r0;  // (the quantised rows are the segment's)
-      aq.q[(size_t)mq * NQ * D + 32 * gq + a8_slot(c32)] = (uint16_t)(as_u32(qv) >> 16);
-      if (c32 == 0) {
-        aq.sx[(size_t)gq * aq.ld + mq] = sx;
-        aq.corr[(size_t)gq * aq.ld + mq] = -136.0f * sum;
-      }
-    }
+    float* orow = att + (size_t)(r0 + 4 * qd + t) * NQ * D + (4 * half + (r & 3)) * D + 64 * w + c32;
+    orow[0] = v[0];
+    orow[32] = v[1];
   }
 }
 
@@ -424,17 +406,17 @@ long long pfa_scratch_floats(int M, int Pb) {
 }
 
 void launch_pfa(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g, int r0,
-                int M, int sliding, hipStream_t st, int hd, const A8Rows& aq) {
+                int M, int sliding, hipStream_t st, int hd) {
   const int Pb = g.pos0 + r0, nq = (M + 3) / 4;
   int ns;
   const int spt = pfa_spt(M, Pb, sliding, &ns);
   float* PM = S + pfa_tiles(M, Pb, sliding) * 1024;
   if (hd == 512) {
     hipLaunchKernelGGL(k_pfa_scores<512>, dim3((M + 7) / 8, ns), dim3(256), 0, st, q, KC, S, PM, g, r0, M, sliding, spt, ns);
-    hipLaunchKernelGGL(k_pfa_out<512>, dim3(nq), dim3(512), 0, st, S, PM, VC, att, g, r0, M, sliding, ns, aq);
+    hipLaunchKernelGGL(k_pfa_out<512>, dim3(nq), dim3(512), 0, st, S, PM, VC, att, g, r0, M, sliding, ns);
   } else {
     hipLaunchKernelGGL(k_pfa_scores<HD>, dim3((M + 7) / 8, ns), dim3(256), 0, st, q, KC, S, PM, g, r0, M, sliding, spt, ns);
-    hipLaunchKernelGGL(k_pfa_out<HD>, dim3(nq), dim3(HD), 0, st, S, PM, VC, att, g, r0, M, sliding, ns, aq);
+    hipLaunchKernelGGL(k_pfa_out<HD>, dim3(nq), dim3(HD), 0, st, S, PM, VC, att, g, r0, M, sliding, ns);
   }
 }
 

@@ -498,10 +498,9 @@ long long pf_score_floats(int M, int Pb) {
   return M > MAXM ? std::max(few, pfa_scratch_floats(M, Pb)) : few;
 }
 void launch_pf_attn(const float* q, const uint16_t* KC, const uint16_t* VC, float* S, float* att, const PfGeom& g,
-                    int r0, int M, int sliding, hipStream_t st, bool staged, int hd, const int* dpos, int maxpos,
-                    const A8Rows& aq) {
+                    int r0, int M, int sliding, hipStream_t st, bool staged, int hd, const int* dpos, int maxpos) {
   if (M > MAXM) {  // a prompt's rows: the matrix-core kernels (no sibling, position from the host, plain rows)
-    launch_pfa(q, KC, VC, S, att, g, r0, M, sliding, st, hd, aq);
+    launch_pfa(q, KC, VC, S, att, g, r0, M, sliding, st, hd);
     return;
   }
   // (dpos: the position comes from device memory; the grid then covers positions below maxpos,
