@@ -183,8 +183,8 @@ __global__ __launch_bounds__(256) void k_head_rescore(HeadScratch hs, HeadDev hd
   }
 }
 
-// full head for the rows whose survivor count exceeds the limit (E:1489-1498); the dec16 row
-// is read once for all MT activation rows.  This pass stores each row's main dot (X3:83-107,
+// full head for the rows whose survivor count exceeds the limit (E:1489-1498); a head row
+// is read once for all of them.  This pass stores each row's main dot (X3:83-107,
 // before the exception deltas); k_head_exc then adds the deltas in order and rounds.
 // the 8 weights of one (row, group pair, lane) entry of the exp3 form (HeadDev::x3sm / x3ix):
 // exponent bytes from the 8-entry codebook by byte permutes, then the bf16 bit patterns
@@ -234,31 +234,34 @@ __global__ void k_x3_pack(HeadDev hd, int V) {
   }
 }
 
+// the rows of the pass that fall back, in order; returns how many (every thread of the block)
 template <int MT>
-__global__ __launch_bounds__(256) void k_head_full(HeadScratch hs, HeadDev hd, const float* __restrict__ h,
-                                                   int V, const int* active) {
-  if (active && *active == 0) return;
-  extern __shared__ float4 lds4[];
-  float4* XH = lds4;
-  float* XR = reinterpret_cast<float*>(lds4 + MT * 48 * 8);
-  bool any = false;
-  bool fb[MT];
+__device__ __forceinline__ int fallback_rows(const HeadScratch& hs, int* rows) {
+  int nf = 0;
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    fb[m] = hs.cnt[m] > HEAD_LIMIT;
-    any |= fb[m];
-  }
-  if (!any) return;
-  stage_h(h, MT, XH, XR);
+  for (int m = 0; m < MT; ++m)
+    if (hs.cnt[m] > HEAD_LIMIT) {
+      if (threadIdx.x == 0) rows[nf] = m;
+      ++nf;
+    }
+  __syncthreads();
+  return nf;
+}
+
+// the dots of every head row with NF of the pass's rows (the last nf of them again in rows nf.., not
+// stored)
+template <int NF>
+__device__ __forceinline__ void head_full_rows(const HeadScratch& hs, const HeadDev& hd, const float4* XH,
+                                               const int* rows, int nf, int V) {
   const uint32_t cblo = reinterpret_cast<const uint32_t*>(hd.cb)[0], cbhi = reinterpret_cast<const uint32_t*>(hd.cb)[1];
   const int j = threadIdx.x & 7, slot = threadIdx.x >> 3, nslots = blockDim.x >> 3;
   for (int n0 = blockIdx.x * nslots; n0 < V; n0 += gridDim.x * nslots) {
     const int n = n0 + slot;
     const bool ok = n < V;
     const int nn = ok ? n : 0;
-    float acc[MT];
+    float acc[NF];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = 0.f;
+    for (int m = 0; m < NF; ++m) acc[m] = 0.f;
     const uint2* ps = hd.x3sm + (size_t)nn * (24 * 8) + j;
     const uint32_t* pi = hd.x3ix + (size_t)nn * (24 * 8) + j;
 #pragma unroll 8
@@ -267,7 +270,7 @@ __global__ __launch_bounds__(256) void k_head_full(HeadScratch hs, HeadDev hd, c
       x3_decode(ps[q * 8], pi[q * 8], cblo, cbhi, wd);
       const float w0 = wd[0], w1 = wd[1], w2 = wd[2], w3 = wd[3], w4 = wd[4], w5 = wd[5], w6 = wd[6], w7 = wd[7];
 #pragma unroll
-      for (int m = 0; m < MT; ++m) {
+      for (int m = 0; m < NF; ++m) {
         const float4 x0 = XH[(m * 48 + 2 * q) * 8 + j], x1 = XH[(m * 48 + 2 * q + 1) * 8 + j];
         float a = acc[m];
         a = fmaf(w0, x0.x, a);
@@ -282,44 +285,79 @@ __global__ __launch_bounds__(256) void k_head_full(HeadScratch hs, HeadDev hd, c
       }
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-      if (!fb[m]) continue;
+    for (int m = 0; m < NF; ++m) {
+      if (m >= nf) break;  // uniform
       float y = acc[m];
       y = y + __shfl_xor(y, 4, 8);
       y = y + __shfl_xor(y, 1, 8);
       y = y + __shfl_xor(y, 2, 8);
-      if (j == 0 && ok) hs.u[(size_t)m * V + n] = y;
+      if (j == 0 && ok) hs.u[(size_t)rows[m] * V + n] = y;
     }
   }
 }
 
+// Only the rows that fall back are staged and take part (one, two, four or MT of them: an unrolled
+// body each).  Bound by the 1.5 bytes a weight for one row (104 us at V = 262144, 5.8 TB/s), by the
+// rows' chains and their LDS words beyond; with every row of the pass in the body, and the rows a
+// second time in LDS for deltas that k_head_exc adds, a 4-row pass of which two fall back took 191 us;
+// with these two 110 (and k_head_exc 32 -> 22).
+template <int MT>
+__global__ __launch_bounds__(256) void k_head_full(HeadScratch hs, HeadDev hd, const float* __restrict__ h,
+                                                   int V, const int* active) {
+  if (active && *active == 0) return;
+  extern __shared__ float4 lds4[];
+  __shared__ int rows[MT];
+  const int nf = fallback_rows<MT>(hs, rows);
+  if (nf == 0) return;
+  const int ns = nf <= 2 ? nf : (nf <= 4 ? min(4, MT) : MT);  // staged rows
+  for (int idx = threadIdx.x; idx < ns * 48 * 8; idx += blockDim.x) {
+    const int j = idx & 7, g = (idx >> 3) % 48, f = idx / (48 * 8);
+    const float* b = h + (size_t)rows[min(f, nf - 1)] * H + g * 32;
+    lds4[idx] = make_float4(b[j], b[16 + j], b[8 + j], b[24 + j]);
+  }
+  __syncthreads();
+  if (nf == 1) {
+    head_full_rows<1>(hs, hd, lds4, rows, nf, V);
+    return;
+  }
+  if constexpr (MT > 2) {
+    if (nf == 2) {
+      head_full_rows<2>(hs, hd, lds4, rows, nf, V);
+      return;
+    }
+  }
+  if constexpr (MT > 4) {
+    if (nf <= 4) {
+      head_full_rows<4>(hs, hd, lds4, rows, nf, V);
+      return;
+    }
+  }
+  if constexpr (MT > 1) head_full_rows<MT>(hs, hd, lds4, rows, nf, V);
+}
+
 // X3:103 / E:565 the exception deltas of each row after its main dot, in list order, then the
-// bf16 rounding of the logit (E:1494); one thread per row.  One partial max per block and row
-// (reduced by the tie kernel).
+// bf16 rounding of the logit (E:1494); one thread per row, for the rows that fall back.  One partial
+// max per block and row (reduced by the tie kernel).
 template <int MT>
 __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, const float* __restrict__ h, int V,
                                                   const int* active) {
   if (active && *active == 0) return;
   extern __shared__ float4 lds4[];
-  float4* XH = lds4;
-  float* XR = reinterpret_cast<float*>(lds4 + MT * 48 * 8);
-  bool any = false;
-  bool fb[MT];
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    fb[m] = hs.cnt[m] > HEAD_LIMIT;
-    any |= fb[m];
-  }
-  if (!any) return;
-  stage_h(h, MT, XH, XR);
+  __shared__ int rows[MT];
+  const int nf = fallback_rows<MT>(hs, rows);
+  if (nf == 0) return;
+  float* XR = reinterpret_cast<float*>(lds4);  // [nf][H]
+  for (int idx = threadIdx.x; idx < nf * (H / 4); idx += blockDim.x)
+    lds4[idx] = reinterpret_cast<const float4*>(h)[(size_t)rows[idx / (H / 4)] * (H / 4) + idx % (H / 4)];
+  __syncthreads();
   float vrun[MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) vrun[m] = -INFINITY;
+  for (int f = 0; f < MT; ++f) vrun[f] = -INFINITY;
   for (int n = blockIdx.x * blockDim.x + threadIdx.x; n < V; n += gridDim.x * blockDim.x) {
     const int e0 = hd.exc_ptr[n], e1 = hd.exc_ptr[n + 1];
     float y[MT];
 #pragma unroll
-    for (int m = 0; m < MT; ++m) y[m] = fb[m] ? hs.u[(size_t)m * V + n] : 0.f;
+    for (int f = 0; f < MT; ++f) y[f] = f < nf ? hs.u[(size_t)rows[f] * V + n] : 0.f;
     for (int e = e0; e < e1; e += 4) {  // four entries per round trip, applied in order
       float dl[4];
       int cl[4];
@@ -333,29 +371,30 @@ __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, co
       for (int k = 0; k < 4; ++k)
         if (e + k < e1) {
 #pragma unroll
-          for (int m = 0; m < MT; ++m) y[m] = fmaf(dl[k], XR[m * H + cl[k]], y[m]);
+          for (int f = 0; f < MT; ++f)
+            if (f < nf) y[f] = fmaf(dl[k], XR[f * H + cl[k]], y[f]);  // (uniform)
         }
     }
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
-      if (fb[m]) {
-        const float v = r16(y[m]);
-        hs.u[(size_t)m * V + n] = v;
-        vrun[m] = fmaxf(vrun[m], v);
+    for (int f = 0; f < MT; ++f)
+      if (f < nf) {
+        const float v = r16(y[f]);
+        hs.u[(size_t)rows[f] * V + n] = v;
+        vrun[f] = fmaxf(vrun[f], v);
       }
   }
   __shared__ float red[256 / 64][MT];
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    float v = vrun[m];
+  for (int f = 0; f < MT; ++f) {
+    float v = vrun[f];
     for (int s = 1; s < 64; s <<= 1) v = fmaxf(v, __shfl_xor(v, s, 64));
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][m] = v;
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][f] = v;
   }
   __syncthreads();
-  if (threadIdx.x < MT) {
+  if ((int)threadIdx.x < nf) {
     float v = -INFINITY;
     for (int w = 0; w < 256 / 64; ++w) v = fmaxf(v, red[w][threadIdx.x]);
-    hs.vpart[(size_t)threadIdx.x * gridDim.x + blockIdx.x] = v;
+    hs.vpart[(size_t)rows[threadIdx.x] * gridDim.x + blockIdx.x] = v;
   }
 }
 
@@ -588,11 +627,8 @@ void head_run(const HeadRun& r, hipStream_t st) {
   mark(PT_HEAD_RESCORE, 1, 0);
   static bool big_lds = false;  // rows 6 to 8 stage more than 64 KB
   if (!big_lds) {
-    const void* fns[] = {reinterpret_cast<const void*>(&k_head_rescore), reinterpret_cast<const void*>(&k_head_full<6>),
-                         reinterpret_cast<const void*>(&k_head_full<7>), reinterpret_cast<const void*>(&k_head_full<8>),
-                         reinterpret_cast<const void*>(&k_head_exc<6>), reinterpret_cast<const void*>(&k_head_exc<7>),
-                         reinterpret_cast<const void*>(&k_head_exc<8>)};
-    for (const void* f : fns) (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)head_lds(MAXM));
+    (void)hipFuncSetAttribute(reinterpret_cast<const void*>(&k_head_rescore), hipFuncAttributeMaxDynamicSharedMemorySize,
+                              (int)head_lds(MAXM));
     big_lds = true;
   }
   hipLaunchKernelGGL(k_head_rescore, dim3(256), dim3(256), head_lds(MT), st, r.hs, r.hd, r.h, MT, r.active);
@@ -601,8 +637,8 @@ void head_run(const HeadRun& r, hipStream_t st) {
   mark(PT_HEAD_FULL, 1, 0);
 #define G4V_HEAD_ROWS(mt)                                                                                       \
   case mt:                                                                                                     \
-    hipLaunchKernelGGL(k_head_full<mt>, gf, dim3(256), head_lds(mt), st, r.hs, r.hd, r.h, V, r.active);       \
-    hipLaunchKernelGGL(k_head_exc<mt>, ge, dim3(256), head_lds(mt), st, r.hs, r.hd, r.h, V, r.active);        \
+    hipLaunchKernelGGL(k_head_full<mt>, gf, dim3(256), (mt) * H * sizeof(float), st, r.hs, r.hd, r.h, V, r.active);       \
+    hipLaunchKernelGGL(k_head_exc<mt>, ge, dim3(256), (mt) * H * sizeof(float), st, r.hs, r.hd, r.h, V, r.active);        \
     break;
   switch (MT) {
     G4V_HEAD_ROWS(1) G4V_HEAD_ROWS(2) G4V_HEAD_ROWS(3) G4V_HEAD_ROWS(4)

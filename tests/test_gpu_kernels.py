@@ -264,6 +264,24 @@ def test_head_full_vocab(orc, dev):
     assert fb[0] == 1 and fb[1] == 1 and fb[2] == 0 and fb[3] == 0
 
 
+@pytest.mark.parametrize("rows", ["r", "ar", "rr", "ara", "rrr", "arra", "rarr", "rrrr"])
+def test_head_fallback_rows(orc, dev, rows):
+    """the full head over the rows that fall back alone (r: every candidate survives the screen; a:
+    few do), one, two and up to four of them, at any places of the call"""
+    V, M = 40960, len(rows)
+    E, P, scr = _head_inputs(orc, V, 6)
+    h = np.where(np.array([c == "r" for c in rows])[:, None], _rows(orc, E, 6, "random", M),
+                 _rows(orc, E, 6, "aligned", M)).astype(np.float32)
+    note(f"head V={V} rows {rows}")
+    dev.head_build(E, V)
+    G, ns, fb = dev.head_argmax(h)
+    for m in range(M):
+        info, surv, sval = orc.head_row(h[m], scr, P)
+        assert G[m] == info.G and ns[m] == info.nsurv, (m, G[m], info.G, ns[m], info.nsurv)
+        assert bool(fb[m]) == (info.nsurv > 30000)
+        assert rows[m] == "a" or fb[m], "meant to fall back"
+
+
 def test_head_exp3_form(orc, dev):
     """the exp3 form the full head streams (x3sm / x3ix, laid out in the fma-lane order of the
     decoded head) carries exactly the oracle's X3 packing (X3:25-43): the codebook, every weight's
