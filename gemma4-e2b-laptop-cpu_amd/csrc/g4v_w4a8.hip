@@ -322,58 +322,63 @@ __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __
   const int tg = blockIdx.x, mi = (tg >= q.t0[1]) + (tg >= q.t0[2]);
   const int t = tg - (mi == 0 ? 0 : (mi == 1 ? q.t0[1] : q.t0[2]));
   const int m0 = blockIdx.y * 16, r = lane & 15, h = lane >> 4;
-  const int G = K / 32, NC = G / 4, NPH = (G + SP_G - 1) / SP_G;
+  const int G = K / 32, NC = G / 4, NPH = ((G + SP_G - 1) / SP_G + 1) & ~1;  // phases, by twos
   const uint4 *tww = q.tw[0], *tss = q.ts[0];
   if (mi == 1) tww = q.tw[1], tss = q.ts[1];
   if (mi == 2) tww = q.tw[2], tss = q.ts[2];
   if (w < 4) {
-    const uint4* wp = tww + (size_t)t * NC * 64 + lane;
-    const uint4* sp = tss + (size_t)t * (G / 8) * 16 + r;
-    const uint16_t* ap = xqb + (size_t)(m0 + r) * K + 8 * h;
-    const float *cp = corr + m0 + 4 * h, *xp = sxt + m0 + 4 * h;
+    const __amdgpu_buffer_rsrc_t wr = buf_rsrc(tww + (size_t)t * NC * 64, (uint32_t)NC * 1024);
+    const __amdgpu_buffer_rsrc_t sr = buf_rsrc(tss + (size_t)t * (G / 8) * 16, (uint32_t)(G / 8) * 256);
+    const __amdgpu_buffer_rsrc_t ar = buf_rsrc(xqb + (size_t)m0 * K, 32u * K);
+    const __amdgpu_buffer_rsrc_t cr = buf_rsrc(corr, (uint32_t)G * Mpad * 4), xr = buf_rsrc(sxt, (uint32_t)G * Mpad * 4);
+    const uint32_t ao = 2u * (r * K + 8 * h), co = 4u * (m0 + 4 * h);
+    auto ld = [](__amdgpu_buffer_rsrc_t rs, uint32_t o) { return __builtin_bit_cast(u32x4_t, buf_load16(rs, o)); };
     struct Ops {
       u32x4_t w, s, a[4];
       f32x4_t c[4], x[4];
     };
-    auto load = [&](Ops& o, int p) {  // chunk 4 p + w (past the last: that one again, not stored)
-      const int c = min(4 * p + w, NC - 1);
-      o.w = *reinterpret_cast<const u32x4_t*>(wp + (size_t)c * 64);
-      o.s = *reinterpret_cast<const u32x4_t*>(sp + (size_t)(c >> 1) * 16);
+    // (No branch between the loads and their uses: a wait behind a join is for every load in flight,
+    // and the phases then took a trip to memory each, 23 us for K = 6144.)
+    auto load = [&](Ops& o, int p) {  // chunk 4 p + w (past the last: that one again, not read)
+      const uint32_t c = min(4 * p + w, NC - 1);
+      o.w = ld(wr, c * 1024 + lane * 16);
+      o.s = ld(sr, (c >> 1) * 256 + r * 16);
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const size_t g = 4 * c + i;
-        o.a[i] = *reinterpret_cast<const u32x4_t*>(ap + 32 * g);
-        o.c[i] = *reinterpret_cast<const f32x4_t*>(cp + g * Mpad);
-        o.x[i] = *reinterpret_cast<const f32x4_t*>(xp + g * Mpad);
+        const uint32_t g = 4 * c + i;
+        o.a[i] = ld(ar, ao + 64 * g);
+        o.c[i] = __builtin_bit_cast(f32x4_t, ld(cr, co + 4 * g * Mpad));
+        o.x[i] = __builtin_bit_cast(f32x4_t, ld(xr, co + 4 * g * Mpad));
       }
     };
     auto form = [&](const Ops& o, int p) {
-      const int c = 4 * p + w;
-      if (c < NC) {  // uniform
-        const bool hi = c & 1;
-        const uint32_t s01 = hi ? o.s[2] : o.s[0], s23 = hi ? o.s[3] : o.s[1];
+      const bool hi = w & 1;  // (the chunk's parity)
+      const uint32_t s01 = hi ? o.s[2] : o.s[0], s23 = hi ? o.s[3] : o.s[1];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t s2 = i < 2 ? s01 : s23;
-          const float sw = as_f32((i & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
-          const f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, o.a[i]),
-                                                                   a8_decode(o.w[i]), o.c[i], 0, 0, 0);
+      for (int i = 0; i < 4; ++i) {
+        const uint32_t s2 = i < 2 ? s01 : s23;
+        const float sw = as_f32((i & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
+        const f32x4_t d = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8_t, o.a[i]),
+                                                                 a8_decode(o.w[i]), o.c[i], 0, 0, 0);
 #pragma unroll
-          for (int k = 0; k < 4; ++k) S[p & 1][4 * w + i][k][lane] = make_float2(d[k], sw * o.x[i][k]);
-        }
+        for (int k = 0; k < 4; ++k) S[p & 1][4 * w + i][k][lane] = make_float2(d[k], sw * o.x[i][k]);
       }
+      __builtin_amdgcn_sched_barrier(0);
       lds_barrier();
     };
     Ops A, B;
     load(A, 0);
+    asm volatile("" ::: "memory");  // (A's loads before B's also through the IR passes)
+    __builtin_amdgcn_sched_barrier(0);
     load(B, 1);
+    __builtin_amdgcn_sched_barrier(0);
     for (int p = 0; p < NPH; p += 2) {
       form(A, p);
       load(A, p + 2);
-      if (p + 1 < NPH) {  // uniform
-        form(B, p + 1);
-        load(B, p + 3);
-      }
+      __builtin_amdgcn_sched_barrier(0);
+      form(B, p + 1);
+      load(B, p + 3);
+      __builtin_amdgcn_sched_barrier(0);
     }
     return;
   }
@@ -382,7 +387,7 @@ __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __
   for (int p = 0; p < NPH; ++p) {
     lds_barrier();  // phase p is formed; the producers go on to the other half
     const float2* s = &S[p & 1][0][i][lane];
-    const int ng = min(SP_G, G - SP_G * p);  // 8 or 16: K % 256 == 0
+    const int ng = min(SP_G, G - SP_G * p);  // 8 or 16 (K % 256 == 0), or none in a last odd phase
     for (int g8 = 0; g8 < ng; g8 += 8)
 #pragma unroll
       for (int g = 0; g < 8; ++g) {
