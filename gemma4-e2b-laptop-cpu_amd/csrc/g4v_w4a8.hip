@@ -128,11 +128,11 @@ template <int MT, int NT, int CG, bool PAIR>
 __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm q, const uint16_t* __restrict__ xqb,
                                                    const float* __restrict__ sxt, const float* __restrict__ corr,
                                                    int M, int Mpad, int K) {
-  constexpr int RB = 16 * MT, ROWB = CG * 64 + 16;  // rows of a block, bytes of a staged row (+ pad)
+  constexpr int RB = 16 * MT;  // rows of a block
   constexpr int NP = MT * CG / 4;                   // 16-byte pieces per thread and step
   constexpr int NC = CG * RB, NCT = (NC + 255) / 256;
   static_assert(MT * CG % 4 == 0 && (CG == 4 || CG == 8), "whole pieces, whole chunks of 4 groups");
-  __shared__ __align__(16) uint8_t As[2][RB * ROWB];
+  __shared__ __align__(16) u32x4_t As[2][64 * MT * CG];  // [MT][CG][16 rows][4 pieces], as in memory
   __shared__ __align__(16) float Cs[2][CG][RB], Ss[2][CG][RB];
   const int lane = threadIdx.x & 63, tid = threadIdx.x, w = threadIdx.x >> 6;
   constexpr int TPW = PAIR ? NT / 2 : NT;           // tiles of a matrix per wave
@@ -168,8 +168,8 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
   auto issue = [&](int st) {
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
-      const int i = tid + 256 * k;  // row i / (4 CG), 16 bytes i % (4 CG) of the step
-      ap[k] = *reinterpret_cast<const u32x4_t*>(xqb + (size_t)(m0 + i / (4 * CG)) * K + 32 * CG * st + 8 * (i % (4 * CG)));
+      const int i = tid + 256 * k;  // 16 bytes i % (64 CG) of the step's groups of row block i / (64 CG)
+      ap[k] = *reinterpret_cast<const u32x4_t*>(xqb + a8_at(K, m0 + 16 * (i / (64 * CG)), CG * st) + 8 * (i % (64 * CG)));
     }
 #pragma unroll
     for (int k = 0; k < NCT; ++k) {
@@ -180,10 +180,7 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
   };
   auto commit = [&](int b) {
 #pragma unroll
-    for (int k = 0; k < NP; ++k) {
-      const int i = tid + 256 * k;
-      *reinterpret_cast<u32x4_t*>(&As[b][(i / (4 * CG)) * ROWB + 16 * (i % (4 * CG))]) = ap[k];
-    }
+    for (int k = 0; k < NP; ++k) As[b][tid + 256 * k] = ap[k];
 #pragma unroll
     for (int k = 0; k < NCT; ++k) {  // (with fewer than 256 entries several threads store the same)
       const int i = (tid + 256 * k) & (NC - 1);
@@ -221,7 +218,7 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
-        const u32x4_t av = *reinterpret_cast<const u32x4_t*>(&As[b][(16 * mt + r) * ROWB + 64 * i + 16 * h]);
+        const u32x4_t av = As[b][((mt * CG + i) * 16 + r) * 4 + h];
         const f32x4_t cin = *reinterpret_cast<const f32x4_t*>(&Cs[b][i][16 * mt + 4 * h]);
         const f32x4_t sx = *reinterpret_cast<const f32x4_t*>(&Ss[b][i][16 * mt + 4 * h]);
         const bf16x8_t A = __builtin_bit_cast(bf16x8_t, av);
@@ -283,7 +280,7 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
         const float q0 = a8_q(v[0], inv, sum), q1 = a8_q(v[1], inv, sum);
         sum = row16_all_sum(sum);
         if (m < M) {
-          uint16_t* d = q.yq.q + (size_t)m * N + 32 * g + a8_slot(r);
+          uint16_t* d = q.yq.q + a8_at(N, m, g) + a8_slot(r);
           d[0] = (uint16_t)(as_u32(q0) >> 16);
           d[16] = (uint16_t)(as_u32(q1) >> 16);
           if (r == 0) {
@@ -312,7 +309,8 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
 // factors sw * sx (a chunk of 4 groups each, operands loaded two phases ahead) into LDS while waves
 // 4..7 run the previous phase's chains, D element i of every lane on wave 4 + i.  A lone wave issues an
 // instruction every ~6 cycles, and in k_w4a8_gemm's loop a tile's group took it ~300 cycles (40 rows,
-// K = 6144: 24 us on 288 waves); here a phase costs its four groups of dots.
+// K = 6144: 24 us on 288 waves); here a phase costs its four groups of dots (17 us; K = 1536, 160 tiles x
+// 3 row blocks: 8.4).  Both sides of its rule (1,024 tiles x row blocks) are in launch_w4a8_gemm_multi.
 constexpr int SP_G = 16;  // groups of a phase
 __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __restrict__ xqb,
                                                     const float* __restrict__ sxt, const float* __restrict__ corr,
@@ -331,7 +329,7 @@ __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __
     const __amdgpu_buffer_rsrc_t sr = buf_rsrc(tss + (size_t)t * (G / 8) * 16, (uint32_t)(G / 8) * 256);
     const __amdgpu_buffer_rsrc_t ar = buf_rsrc(xqb + (size_t)m0 * K, 32u * K);
     const __amdgpu_buffer_rsrc_t cr = buf_rsrc(corr, (uint32_t)G * Mpad * 4), xr = buf_rsrc(sxt, (uint32_t)G * Mpad * 4);
-    const uint32_t ao = 2u * (r * K + 8 * h), co = 4u * (m0 + 4 * h);
+    const uint32_t ao = 64 * r + 16 * h, co = 4u * (m0 + 4 * h);
     auto ld = [](__amdgpu_buffer_rsrc_t rs, uint32_t o) { return __builtin_bit_cast(u32x4_t, buf_load16(rs, o)); };
     struct Ops {
       u32x4_t w, s, a[4];
@@ -346,7 +344,7 @@ __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const uint32_t g = 4 * c + i;
-        o.a[i] = ld(ar, ao + 64 * g);
+        o.a[i] = ld(ar, ao + 1024 * g);
         o.c[i] = __builtin_bit_cast(f32x4_t, ld(cr, co + 4 * g * Mpad));
         o.x[i] = __builtin_bit_cast(f32x4_t, ld(xr, co + 4 * g * Mpad));
       }
@@ -428,7 +426,7 @@ __global__ __launch_bounds__(1024) void k_w4a8_dec(A8Dec m, const uint16_t* __re
   const int G = K / 32;
   const uint4* wp = tw + (size_t)t * (G / 4) * 64 + lane;  // chunk c at + 64 c
   const uint4* sp = ts + (size_t)t * (G / 8) * 16 + r;     // scales of groups 8 c8 .. at + 16 c8
-  const uint16_t* ap = xqb + (size_t)r * K + 8 * h;         // group g at + 32 g
+  const uint16_t* ap = xqb + a8_at(K, r, 0) + 8 * h;        // group g at + 512 g
   const int mrow = 4 * h;
   const int cm = tid >> 4, cr = tid & 15;                   // chain lane: row cm, column cr
   const int cl = ((cm >> 2) << 4) | cr, ci = cm & 3;
@@ -447,7 +445,7 @@ __global__ __launch_bounds__(1024) void k_w4a8_dec(A8Dec m, const uint16_t* __re
         const int gi = 4 * (c & 1) + i;
         const uint32_t s2 = gi < 2 ? scur.x : (gi < 4 ? scur.y : (gi < 6 ? scur.z : scur.w));
         const float sw = as_f32((gi & 1) ? (s2 & 0xFFFF0000u) : (s2 << 16));
-        const uint4 av = *reinterpret_cast<const uint4*>(ap + 32 * (size_t)g);
+        const uint4 av = *reinterpret_cast<const uint4*>(ap + 512 * (size_t)g);
         const float4 crv = *reinterpret_cast<const float4*>(corr + (size_t)g * Mpad + mrow);
         const float4 sx = *reinterpret_cast<const float4*>(sxt + (size_t)g * Mpad + mrow);
         const f32x4_t cin = {crv.x, crv.y, crv.z, crv.w};
