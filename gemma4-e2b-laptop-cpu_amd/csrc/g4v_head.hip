@@ -234,25 +234,26 @@ __global__ void k_x3_pack(HeadDev hd, int V) {
   }
 }
 
-// the rows of the pass that fall back, in order; returns how many (every thread of the block)
+// the rows of the pass that fall back, in order (rw[f], f < the returned count; 0 past it): uniform
+// values, no exchange through LDS (a list there cost the head of one row 3 us of 202)
 template <int MT>
-__device__ __forceinline__ int fallback_rows(const HeadScratch& hs, int* rows) {
-  int nf = 0;
+__device__ __forceinline__ int fallback_rows(const HeadScratch& hs, int (&rw)[MT]) {
+  uint32_t mask = 0;
 #pragma unroll
-  for (int m = 0; m < MT; ++m)
-    if (hs.cnt[m] > HEAD_LIMIT) {
-      if (threadIdx.x == 0) rows[nf] = m;
-      ++nf;
-    }
-  __syncthreads();
+  for (int m = 0; m < MT; ++m) mask |= (hs.cnt[m] > HEAD_LIMIT ? 1u : 0u) << m;
+  const int nf = __builtin_popcount(mask);
+#pragma unroll
+  for (int f = 0; f < MT; ++f) {
+    rw[f] = mask ? __builtin_ctz(mask) : 0;
+    mask &= mask - 1u;
+  }
   return nf;
 }
 
-// the dots of every head row with NF of the pass's rows (the last nf of them again in rows nf.., not
-// stored)
-template <int NF>
+// the dots of every head row with NF of the pass's rows (nf of them, the others not stored)
+template <int NF, int MT>
 __device__ __forceinline__ void head_full_rows(const HeadScratch& hs, const HeadDev& hd, const float4* XH,
-                                               const int* rows, int nf, int V) {
+                                               const int (&rw)[MT], int nf, int V) {
   const uint32_t cblo = reinterpret_cast<const uint32_t*>(hd.cb)[0], cbhi = reinterpret_cast<const uint32_t*>(hd.cb)[1];
   const int j = threadIdx.x & 7, slot = threadIdx.x >> 3, nslots = blockDim.x >> 3;
   for (int n0 = blockIdx.x * nslots; n0 < V; n0 += gridDim.x * nslots) {
@@ -291,7 +292,7 @@ __device__ __forceinline__ void head_full_rows(const HeadScratch& hs, const Head
       y = y + __shfl_xor(y, 4, 8);
       y = y + __shfl_xor(y, 1, 8);
       y = y + __shfl_xor(y, 2, 8);
-      if (j == 0 && ok) hs.u[(size_t)rows[m] * V + n] = y;
+      if (j == 0 && ok) hs.u[(size_t)rw[m] * V + n] = y;
     }
   }
 }
@@ -306,33 +307,37 @@ __global__ __launch_bounds__(256) void k_head_full(HeadScratch hs, HeadDev hd, c
                                                    int V, const int* active) {
   if (active && *active == 0) return;
   extern __shared__ float4 lds4[];
-  __shared__ int rows[MT];
-  const int nf = fallback_rows<MT>(hs, rows);
+  int rw[MT];
+  const int nf = fallback_rows<MT>(hs, rw);
   if (nf == 0) return;
   const int ns = nf <= 2 ? nf : (nf <= 4 ? min(4, MT) : MT);  // staged rows
-  for (int idx = threadIdx.x; idx < ns * 48 * 8; idx += blockDim.x) {
-    const int j = idx & 7, g = (idx >> 3) % 48, f = idx / (48 * 8);
-    const float* b = h + (size_t)rows[min(f, nf - 1)] * H + g * 32;
-    lds4[idx] = make_float4(b[j], b[16 + j], b[8 + j], b[24 + j]);
+#pragma unroll
+  for (int f = 0; f < MT; ++f) {
+    if (f >= ns) break;  // uniform (rows past nf: row 0, not stored)
+    for (int idx = threadIdx.x; idx < 48 * 8; idx += blockDim.x) {
+      const int j = idx & 7, g = idx >> 3;
+      const float* b = h + (size_t)rw[f] * H + g * 32;
+      lds4[f * 48 * 8 + idx] = make_float4(b[j], b[16 + j], b[8 + j], b[24 + j]);
+    }
   }
   __syncthreads();
   if (nf == 1) {
-    head_full_rows<1>(hs, hd, lds4, rows, nf, V);
+    head_full_rows<1>(hs, hd, lds4, rw, nf, V);
     return;
   }
   if constexpr (MT > 2) {
     if (nf == 2) {
-      head_full_rows<2>(hs, hd, lds4, rows, nf, V);
+      head_full_rows<2>(hs, hd, lds4, rw, nf, V);
       return;
     }
   }
   if constexpr (MT > 4) {
     if (nf <= 4) {
-      head_full_rows<4>(hs, hd, lds4, rows, nf, V);
+      head_full_rows<4>(hs, hd, lds4, rw, nf, V);
       return;
     }
   }
-  if constexpr (MT > 1) head_full_rows<MT>(hs, hd, lds4, rows, nf, V);
+  if constexpr (MT > 1) head_full_rows<MT>(hs, hd, lds4, rw, nf, V);
 }
 
 // X3:103 / E:565 the exception deltas of each row after its main dot, in list order, then the
@@ -343,12 +348,15 @@ __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, co
                                                   const int* active) {
   if (active && *active == 0) return;
   extern __shared__ float4 lds4[];
-  __shared__ int rows[MT];
-  const int nf = fallback_rows<MT>(hs, rows);
+  int rw[MT];
+  const int nf = fallback_rows<MT>(hs, rw);
   if (nf == 0) return;
   float* XR = reinterpret_cast<float*>(lds4);  // [nf][H]
-  for (int idx = threadIdx.x; idx < nf * (H / 4); idx += blockDim.x)
-    lds4[idx] = reinterpret_cast<const float4*>(h)[(size_t)rows[idx / (H / 4)] * (H / 4) + idx % (H / 4)];
+#pragma unroll
+  for (int f = 0; f < MT; ++f)
+    if (f < nf)  // (uniform)
+      for (int idx = threadIdx.x; idx < H / 4; idx += blockDim.x)
+        lds4[f * (H / 4) + idx] = reinterpret_cast<const float4*>(h)[(size_t)rw[f] * (H / 4) + idx];
   __syncthreads();
   float vrun[MT];
 #pragma unroll
@@ -357,7 +365,7 @@ __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, co
     const int e0 = hd.exc_ptr[n], e1 = hd.exc_ptr[n + 1];
     float y[MT];
 #pragma unroll
-    for (int f = 0; f < MT; ++f) y[f] = f < nf ? hs.u[(size_t)rows[f] * V + n] : 0.f;
+    for (int f = 0; f < MT; ++f) y[f] = f < nf ? hs.u[(size_t)rw[f] * V + n] : 0.f;
     for (int e = e0; e < e1; e += 4) {  // four entries per round trip, applied in order
       float dl[4];
       int cl[4];
@@ -379,7 +387,7 @@ __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, co
     for (int f = 0; f < MT; ++f)
       if (f < nf) {
         const float v = r16(y[f]);
-        hs.u[(size_t)rows[f] * V + n] = v;
+        hs.u[(size_t)rw[f] * V + n] = v;
         vrun[f] = fmaxf(vrun[f], v);
       }
   }
@@ -391,11 +399,13 @@ __global__ __launch_bounds__(256) void k_head_exc(HeadScratch hs, HeadDev hd, co
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][f] = v;
   }
   __syncthreads();
-  if ((int)threadIdx.x < nf) {
-    float v = -INFINITY;
-    for (int w = 0; w < 256 / 64; ++w) v = fmaxf(v, red[w][threadIdx.x]);
-    hs.vpart[(size_t)rows[threadIdx.x] * gridDim.x + blockIdx.x] = v;
-  }
+#pragma unroll
+  for (int f = 0; f < MT; ++f)
+    if ((int)threadIdx.x == f && f < nf) {
+      float v = -INFINITY;
+      for (int w = 0; w < 256 / 64; ++w) v = fmaxf(v, red[w][f]);
+      hs.vpart[(size_t)rw[f] * gridDim.x + blockIdx.x] = v;
+    }
 }
 
 // lowest index satisfying the tie rule, over survivors or over the full-head logits
