@@ -9,7 +9,8 @@
 // every one of 8192 outputs tried, in normal, subnormal-result and subnormal-operand ranges), so
 // two of them chained from 0 form a lane chain's four-term a for 32 rows x 32 outputs.  (From +0
 // instead of the reference's plain first product only the sign of a zero a can differ, and
-// fma(+-0, sc, row) leaves row as it is: row starts at +0 and a sum is -0 only of two -0.)
+// fma(+-0, sc, row) leaves row as it is: row starts at +0, and it is -0 only after a product a sc
+// below 2^-150 of negative sign, where the sign of an output that is zero is all that can change.)
 // Operands need no shuffling: instruction k = lane / 32 takes x[32g + 16k + 2j] (then + 1) and
 // nibble lo (then hi) of byte 8k + j, so a lane holds consecutive floats of its row and
 // consecutive bytes of its output's group, as the W4A8 operand tiles (k_tile_a8) store them.
@@ -23,7 +24,7 @@
 // prompts still fill the SIMDs.  The block's rows go through LDS four groups at a time (the eight
 // waves read different floats of the same lines), double-buffered, one LDS barrier per step.
 // Measured (333-row prompt, 35 layers, exact float): q/k/v, o and down 69 us, gate / up 181 us on
-// average, the prompt 212.5 -> 18.6 ms (the 8-row GEMV took 42 launches of 8 to 42 us a product).
+// average, the prompt 212.5 -> 18.6 ms (16.5 with its attention on the matrix cores; the 8-row GEMV took 42 launches of 8 to 42 us a product).
 // Row pitch 130 floats: the 32 rows of an 8-byte read fall on 64 different banks.
 #include "g4v_internal.h"
 

@@ -310,7 +310,7 @@ __global__ __launch_bounds__(256, MT * NT >= 16 ? 2 : 3) void k_w4a8_gemm(A8Gemm
 // 4..7 run the previous phase's chains, D element i of every lane on wave 4 + i.  A lone wave issues an
 // instruction every ~6 cycles, and in k_w4a8_gemm's loop a tile's group took it ~300 cycles (40 rows,
 // K = 6144: 24 us on 288 waves); here a phase costs its four groups of dots (17 us; K = 1536, 160 tiles x
-// 3 row blocks: 8.4).  Both sides of its rule (1,024 tiles x row blocks) are in launch_w4a8_gemm_multi.
+// 3 row blocks: 8.4).
 constexpr int SP_G = 16;  // groups of a phase
 __global__ __launch_bounds__(512) void k_w4a8_split(A8Gemm q, const uint16_t* __restrict__ xqb,
                                                     const float* __restrict__ sxt, const float* __restrict__ corr,
@@ -506,8 +506,11 @@ int launch_w4a8_gemm_multi(const A8Gemm& q_in, int n, bool pair, const uint16_t*
     else launch_gemm<1, 4, 4, true>(q, xqb, sxt, corr, M, K, st);
     return 1;
   }
+  // A tile per block of eight waves while every block has a place at once (two a CU at 128 VGPRs, 64 KB
+  // of LDS): prompts of 32 / 64 rows 3.1 / 3.6 ms with every product on it, 3.7 / 3.8 with none; of 96 /
+  // 128 / 160 rows (576 to 960 blocks for o and down) 4.3 / 4.5 / 5.1 ms with, 4.0 / 4.2 / 4.2 without.
   if (by4 && M > 64 && waves1 > 8192) launch_gemm<4, 4, 4, false>(q, xqb, sxt, corr, M, K, st);
-  else if (waves1 <= 1024)
+  else if (waves1 <= 512)
     hipLaunchKernelGGL(k_w4a8_split, dim3(tiles, (M + 15) / 16), dim3(512), 0, st, q, xqb, sxt, corr, M, w4a8_mpad(M), K);
   else launch_gemm<1, 1, 8, false>(q, xqb, sxt, corr, M, K, st);
   return 1;

@@ -56,10 +56,10 @@ def test_w4a8_bit_exact(orc, dev, M, N, K):
     assert same(y, yo), first_diff(y, yo)
 
 
-# the prompt products of more than 8 rows: a tile per eight waves (up to 1,024 tiles x row blocks: half,
+# the prompt products of more than 8 rows: a tile per eight waves (up to 512 tiles x row blocks: half,
 # one, one and a half and more phases of 16 groups, row blocks with one row), a tile per wave, and
 # 64 x 64 blocks (more than 64 rows and 8,192 of those, columns by 64) with remainders
-A8_PROMPT = [(9, 16, 256), (16, 48, 512), (17, 16, 768), (33, 1536, 1280), (40, 512, 6144), (64, 4096, 256),
+A8_PROMPT = [(9, 16, 256), (16, 48, 512), (17, 16, 768), (33, 1536, 1280), (40, 512, 6144), (64, 2048, 256), (65, 2048, 256),
              (65, 4096, 256), (65, 4096, 2304), (65, 26304, 256), (129, 17536, 768), (65, 26320, 256)]
 
 
